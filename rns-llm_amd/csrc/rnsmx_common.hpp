@@ -50,4 +50,19 @@ inline bool packed_accumulator_fits(const rnsmx_moduli_t &mods, int64_t k) {
   return k * 256 * static_cast<int64_t>(max_half(mods)) + 255 <= 0x7FFFFFFFLL;
 }
 
+// Constants of the fractional reconstruction (frac_sum, rnsmx_gemm.hpp) of a
+// set of up to 6 moduli: k_c = (P_p / m_c)^-1 mod m_c, centered, for the
+// prefix of the first p channels, as bytes (kprefix[p], channel c in byte
+// c % 4 of word c / 4), and k_c / m_c of the full set in rows: row 0 to
+// multiples of 2^-20, then either the rest to 53 bits (rest1), or row 1 to
+// multiples of 2^-40 and the rest after it to 53 bits (rest2).
+struct FracSet {
+  double row0[6], rest1[6], row1[6], rest2[6];
+  double p, half, turn;  // P, (P - 1) >> 1 and (half + 1/4) / P of the set
+  uint32_t kprefix[7][2];
+};
+// Kept per thread for the set last asked for, compared by value: the inverses
+// would cost every launch a few hundred nanoseconds.
+const FracSet &frac_set(const rnsmx_moduli_t &mods);
+
 }  // namespace rnsmx

@@ -57,6 +57,18 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 // block (the runtime writes the argument block for every launch, and its
 // host cost grows with the size: 0.9 KB measured 1 us more per launch than
 // 16 bytes).
+//
+// frac: the rows of the fractional reconstruction (frac_sum) of the full set,
+// kFracParts of them; p_full the set's product and turn its starting phase;
+// kprefix[p]: the bytes k_c (centered) of the first p channels, from which
+// the kernel derives the rows of a shorter prefix (prefix_frac).
+template <int RCAP>
+constexpr int kFracParts = RCAP <= 4 ? 2 : RCAP <= 6 ? 3 : 0;
+template <int RCAP>
+constexpr bool kFrac = kFracParts<RCAP> > 0;
+
+constexpr double kRoundMagic = 6755399441055744.0;  // 1.5 * 2^52: one unit in its last place is 1
+
 template <int RCAP>
 struct GemmMods {
   int32_t channels;
@@ -67,6 +79,9 @@ struct GemmMods {
   uint32_t qk8[RCAP];
   uint32_t ucoef[RCAP][RCAP];
   int64_t prefix[RCAP + 1];
+  double frac[kFrac<RCAP> ? kFracParts<RCAP> : 1][kFrac<RCAP> ? RCAP : 1];
+  double p_full, turn, magic_p;
+  uint32_t kprefix[kFrac<RCAP> ? RCAP + 1 : 1][2];
 };
 
 // Arguments of one GEMM launch.  The host fills GemmArgs (with the full
@@ -127,6 +142,22 @@ inline GemmArgsK<RCAP> compact_args(const GemmArgs &g) {
     for (int j = 0; j < RCAP && j < RNSMX_MAX_CHANNELS; ++j) k.mods.ucoef[j][c] = f.ucoef[j][c];
   }
   for (int c = 0; c <= RCAP && c <= RNSMX_MAX_CHANNELS; ++c) k.mods.prefix[c] = f.prefix[c];
+  if constexpr (kFrac<RCAP>) {
+    const FracSet &fs = frac_set(f);
+    k.mods.p_full = fs.p;
+    k.mods.turn = fs.turn;
+    k.mods.magic_p = kRoundMagic - fs.half;
+    for (int c = 0; c < RCAP; ++c) {
+      k.mods.frac[0][c] = fs.row0[c];
+      if constexpr (kFracParts<RCAP> == 2) {
+        k.mods.frac[1][c] = fs.rest1[c];
+      } else {
+        k.mods.frac[1][c] = fs.row1[c];
+        k.mods.frac[2][c] = fs.rest2[c];
+      }
+    }
+    std::memcpy(k.mods.kprefix, fs.kprefix, sizeof(k.mods.kprefix));
+  }
   return k;
 }
 
@@ -201,6 +232,15 @@ __device__ __forceinline__ RNSMX_KARG(T) & kernel_args() {
 }
 template <int RCAP>
 using KArgs = RNSMX_KARG(GemmArgsK<RCAP>);
+// The same arguments through a pointer the compiler cannot see through, so
+// reads after this point are not moved ahead of it (where they would hold
+// registers through a loop that has none to spare).
+template <int RCAP>
+__device__ __forceinline__ KArgs<RCAP> &args_from_here(KArgs<RCAP> &g) {
+  KArgs<RCAP> *p = &g;
+  asm volatile("" : "+s"(p));
+  return *p;
+}
 
 // Touches the first BYTES of the argument block, one read per 64-byte line,
 // in one round at kernel entry.  The block is written for each launch, so
@@ -409,21 +449,32 @@ __device__ __forceinline__ int active_channels(KArgs<RCAP> &g, int64_t *red, int
     }
   }
   __syncthreads();
-  return *bcast;
+  return __builtin_amdgcn_readfirstlane(*bcast);
 }
 
-// Everything the epilogue needs, read from the kernel arguments once per
-// kernel and pinned in scalar registers (pin_epi) right after the first
-// global loads are issued: left to itself the compiler re-issues these
-// scalar loads at their first use in the epilogue, where each dependent
-// round of scalar-cache misses is exposed.
+// The integer constants of the residue and mixed-radix arithmetic
+// (reduce_acc, garner_value, garner_from_sums).
 template <int RCAP>
-struct Epi {
+struct IntConsts {
   uint32_t m[RCAP], m24[RCAP], c16[RCAP], bias[RCAP], qinv[RCAP], qk8[RCAP];
   int32_t negm[RCAP], qk16[RCAP];
   uint32_t u[RCAP][RCAP];  // u[j][c], j < c
   int64_t prefix[RCAP + 1];
   int64_t p_act;  // prefix[c_act], the modulus of the signed correction
+};
+
+// Everything the epilogue needs, read from the kernel arguments once per
+// kernel and pinned in scalar registers (pin_epi) right after the first
+// global loads are issued: left to itself the compiler re-issues these
+// scalar loads at their first use in the epilogue, where each dependent
+// round of scalar-cache misses is exposed.  The integer constants are read
+// here only past 6 channels; elsewhere by the K split's exchange, the one
+// path that needs them (int_consts).
+template <int RCAP>
+struct Epi {
+  double f[kFrac<RCAP> ? kFracParts<RCAP> : 1][RCAP];  // rows of frac_sum for the active prefix
+  double p, turn, magic;
+  IntConsts<RCAP> ic;  // past 6 channels only
   int32_t out_dtype;
   int64_t out_ld;
   void *out;
@@ -432,10 +483,9 @@ struct Epi {
   float a_scale;
 };
 
-// Moduli constants of Epi from a moduli block (kernel arguments or a
-// by-value copy).
+// IntConsts from a moduli block (kernel arguments or a by-value copy).
 template <int RCAP, typename Mods>
-__device__ __forceinline__ void fill_moduli(Epi<RCAP> &e, const Mods &mods, int c_act) {
+__device__ __forceinline__ void fill_moduli(IntConsts<RCAP> &e, const Mods &mods, int c_act) {
   static_for<RCAP>([&](auto C) {
     constexpr int c = decltype(C)::value;
     const uint32_t m = static_cast<uint32_t>(mods.moduli[c]), magic = mods.magic[c];
@@ -455,17 +505,6 @@ __device__ __forceinline__ void fill_moduli(Epi<RCAP> &e, const Mods &mods, int 
   e.p_act = prefix_at<RCAP>(mods, c_act);
 }
 
-template <int RCAP>
-__device__ __forceinline__ void load_epi(KArgs<RCAP> &g, Epi<RCAP> &e, int c_act) {
-  fill_moduli<RCAP>(e, g.mods, c_act);
-  e.out_dtype = g.out_dtype;
-  e.out_ld = g.out_ld;
-  e.out = g.out;
-  e.w_scale = g.w_scale;
-  e.bias_ptr = g.bias;
-  e.a_scale = g.out_dtype != RNSMX_INT64 ? *g.a_scale : 0.0f;
-}
-
 template <typename T>
 __device__ __forceinline__ void pin_sgpr(T &v) {
   static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32- or 64-bit values only");
@@ -483,24 +522,170 @@ __device__ __forceinline__ void pin_sgpr(T &v) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Reconstruction by fractions (up to 6 channels).  By the Chinese remainder
+// theorem the integer y with y = v_c (mod m_c) satisfies y / P = sum_c v_c
+// k_c / m_c (mod 1), k_c = (P / m_c)^-1 mod m_c: one weighted sum of the
+// int32 channel sums, with no residue, digit or dependent chain per channel.
+// The weights are split into rows so that double arithmetic is exact where
+// it has to be (|k_c / m_c| <= 1/2, |v_c| <= 2^31):
+//   row 0  k_c / m_c rounded to multiples of 2^-20: every product and
+//          partial sum is a multiple of 2^-20 of at most 6 * 2^30, so under
+//          53 bits and exact, and so is its fraction z in [0, 1).
+//   up to 4 channels (P < 2^32), row 1  the rest (at most 2^-21) to 53
+//          bits: products of at most 2^10 on top of `turn`, five roundings
+//          of at most 2^-42 each and the row's own error (2^-41): 2^-39.
+//   up to 6 channels (P < 2^48), row 1  the rest rounded to multiples of
+//          2^-40: again exact (terms of at most 2^10), the fraction taken;
+//          row 2  what is left (at most 2^-41) to 53 bits: products of at
+//          most 2^-10 on top of `turn`, six roundings of at most 2^-54 and
+//          one of 2^-53: under 2^-51.
+// turn = (h + 1/4) / P with h = (P - 1) >> 1 turns the centered range (the
+// signed correction of the reference: y <= P / 2 stays, larger x become x -
+// P) onto [0, 1): z + turn = (y + h + 1/4) / P (mod 1), and the right side
+// lies at least 1 / (4 P) inside [0, 1), further than the error above, so
+// the fraction taken last is of the right turn.  Times P its error is below
+// 1/8, so y + h + 1/4 rounds to y + h: the last fma adds 1.5 * 2^52 - h,
+// where units in the last place are 1, and leaves y in the low bits in two's
+// complement.
+// Against the mixed-radix digits in 24-bit integers (garner_from_sums): 16
+// instructions per element for 4 channels instead of about 55, 29 instead of
+// about 110 for 6; each issues in 4 cycles on gfx950, fp64 included.
+// ---------------------------------------------------------------------------
 template <int RCAP>
-__device__ __forceinline__ void pin_epi(Epi<RCAP> &e) {
+__device__ __forceinline__ double frac_sum(const Epi<RCAP> &e, const int32_t (&v)[RCAP]) {
+  double x[RCAP];
+  static_for<RCAP>([&](auto C) { x[decltype(C)::value] = static_cast<double>(v[decltype(C)::value]); });
+  constexpr int L = kFracParts<RCAP> - 1;
+  double z = x[0] * e.f[0][0];
+  static_for<RCAP - 1>([&](auto C) { z = __builtin_fma(x[decltype(C)::value + 1], e.f[0][decltype(C)::value + 1], z); });
+  z = __builtin_amdgcn_fract(z);
+  static_for<L - 1>([&](auto R) {
+    static_for<RCAP>([&](auto C) {
+      z = __builtin_fma(x[decltype(C)::value], e.f[decltype(R)::value + 1][decltype(C)::value], z);
+    });
+    z = __builtin_amdgcn_fract(z);
+  });
+  double s = e.turn;
+  static_for<RCAP>([&](auto C) { s = __builtin_fma(x[decltype(C)::value], e.f[L][decltype(C)::value], s); });
+  return __builtin_fma(__builtin_amdgcn_fract(z + s), e.p, e.magic);
+}
+
+// The integer y held by 1.5 * 2^52 + y: up to 4 channels |y| <= 2^31.
+template <int RCAP>
+__device__ __forceinline__ int64_t frac_int(double t) {
+  const uint64_t bits = __builtin_bit_cast(uint64_t, t);
+  const uint32_t lo = static_cast<uint32_t>(bits);
+  const uint32_t hi = RCAP <= 4 ? static_cast<uint32_t>(static_cast<int32_t>(lo) >> 31)
+                                : static_cast<uint32_t>(bits >> 32) - 0x43380000u;
+  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// A wave-uniform double in vector registers, moved to scalar ones.  The empty
+// assembly hides that it is uniform: the compiler drops a readfirstlane of a
+// value it knows to be, and vector results then stay in vector registers.
+__device__ __forceinline__ void move_to_sgpr(double &v) {
+  const uint64_t w = __builtin_bit_cast(uint64_t, v);
+  uint32_t lo = static_cast<uint32_t>(w), hi = static_cast<uint32_t>(w >> 32);
+  asm volatile("" : "+v"(lo), "+v"(hi));
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  v = __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// The rows of frac_sum for a prefix shorter than the set (adaptive calls):
+// from the bytes k_c with the roundings of the host's (frac_set); once per
+// wave.  x - h m is exact (h has 20 bits, m 8), so each row's rest is too.
+// Every channel's rows go to scalar registers before the next channel's are
+// formed: all at once, the divisions' registers would lower the occupancy of
+// the kernels that run this beside their first loads or their accumulators.
+template <int RCAP>
+__device__ __forceinline__ void prefix_frac(KArgs<RCAP> &g, Epi<RCAP> &e, int c_act) {
+  uint32_t k0 = g.mods.kprefix[0][0], k1 = g.mods.kprefix[0][1];
+  static_for<RCAP + 1>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    if (c_act == i) {
+      k0 = g.mods.kprefix[i][0];
+      k1 = g.mods.kprefix[i][1];
+    }
+  });
   static_for<RCAP>([&](auto C) {
     constexpr int c = decltype(C)::value;
-    pin_sgpr(e.m[c]);
-    pin_sgpr(e.m24[c]);
-    pin_sgpr(e.c16[c]);
-    pin_sgpr(e.bias[c]);
-    pin_sgpr(e.negm[c]);
-    pin_sgpr(e.qinv[c]);
-    if constexpr (c > 0) {
-      pin_sgpr(e.qk16[c]);
-      pin_sgpr(e.qk8[c]);
-    }
-    static_for<c>([&](auto J) { pin_sgpr(e.u[decltype(J)::value][c]); });
+    const uint32_t word = c < 4 ? k0 : k1;
+    double rest = static_cast<double>(static_cast<int8_t>((word >> (8 * (c % 4))) & 0xFFu));
+    const double m = static_cast<double>(max(g.mods.moduli[c], 1u));  // 0 past the set, whose k is 0
+    double scale = 1048576.0;
+    static_for<kFracParts<RCAP> - 1>([&](auto R) {
+      const double h = __builtin_rint(rest / m * scale) / scale;
+      e.f[decltype(R)::value][c] = h;
+      move_to_sgpr(e.f[decltype(R)::value][c]);
+      rest = __builtin_fma(-h, m, rest);
+      scale *= 1048576.0;
+    });
+    e.f[kFracParts<RCAP> - 1][c] = rest / m;
+    move_to_sgpr(e.f[kFracParts<RCAP> - 1][c]);
   });
-  static_for<RCAP + 1>([&](auto C) { pin_sgpr(e.prefix[decltype(C)::value]); });
-  pin_sgpr(e.p_act);
+  const int64_t p = prefix_at<RCAP>(g.mods, c_act);
+  const double half = static_cast<double>((p - 1) >> 1);
+  e.p = static_cast<double>(p);
+  e.turn = (half + 0.25) / e.p;
+  e.magic = kRoundMagic - half;
+  move_to_sgpr(e.p);
+  move_to_sgpr(e.turn);
+  move_to_sgpr(e.magic);
+}
+
+// PREFIX: derive the rows of a shorter prefix here (else the caller has, ahead
+// of loads whose registers the derivation should not share).
+template <int RCAP, bool PREFIX = true>
+__device__ __forceinline__ void load_epi(KArgs<RCAP> &g, Epi<RCAP> &e, int c_act) {
+  if constexpr (kFrac<RCAP>) {
+    if (c_act == g.mods.channels) {
+      static_for<kFracParts<RCAP>>([&](auto R) {
+        static_for<RCAP>([&](auto C) { e.f[R][C] = g.mods.frac[decltype(R)::value][decltype(C)::value]; });
+      });
+      e.p = g.mods.p_full;
+      e.turn = g.mods.turn;
+      e.magic = g.mods.magic_p;
+    } else if constexpr (PREFIX) {
+      prefix_frac<RCAP>(g, e, c_act);
+    }
+  } else {
+    fill_moduli<RCAP>(e.ic, g.mods, c_act);
+  }
+  e.out_dtype = g.out_dtype;
+  e.out_ld = g.out_ld;
+  e.out = g.out;
+  e.w_scale = g.w_scale;
+  e.bias_ptr = g.bias;
+  e.a_scale = g.out_dtype != RNSMX_INT64 ? *g.a_scale : 0.0f;
+}
+
+template <int RCAP>
+__device__ __forceinline__ void pin_epi(Epi<RCAP> &e) {
+  if constexpr (kFrac<RCAP>) {
+    static_for<kFracParts<RCAP>>([&](auto R) { static_for<RCAP>([&](auto C) { pin_sgpr(e.f[R][C]); }); });
+    pin_sgpr(e.p);
+    pin_sgpr(e.turn);
+    pin_sgpr(e.magic);
+  } else {
+    static_for<RCAP>([&](auto C) {
+      constexpr int c = decltype(C)::value;
+      pin_sgpr(e.ic.m[c]);
+      pin_sgpr(e.ic.m24[c]);
+      pin_sgpr(e.ic.c16[c]);
+      pin_sgpr(e.ic.bias[c]);
+      pin_sgpr(e.ic.negm[c]);
+      pin_sgpr(e.ic.qinv[c]);
+      if constexpr (c > 0) {
+        pin_sgpr(e.ic.qk16[c]);
+        pin_sgpr(e.ic.qk8[c]);
+      }
+      static_for<c>([&](auto J) { pin_sgpr(e.ic.u[decltype(J)::value][c]); });
+    });
+    static_for<RCAP + 1>([&](auto C) { pin_sgpr(e.ic.prefix[decltype(C)::value]); });
+    pin_sgpr(e.ic.p_act);
+  }
   pin_sgpr(e.out_ld);
   pin_sgpr(e.out);
   pin_sgpr(e.out_dtype);
@@ -509,13 +694,26 @@ __device__ __forceinline__ void pin_epi(Epi<RCAP> &e) {
   pin_sgpr(e.bias_ptr);
 }
 
+// The integer constants for a path that needs them: read here where
+// load_epi did not.
+template <int RCAP>
+__device__ __forceinline__ IntConsts<RCAP> int_consts(KArgs<RCAP> &g, const Epi<RCAP> &e, int c_act) {
+  if constexpr (kFrac<RCAP>) {
+    IntConsts<RCAP> ic;
+    fill_moduli<RCAP>(ic, g.mods, c_act);
+    return ic;
+  } else {
+    return e.ic;
+  }
+}
+
 // Canonical residue of one int32 accumulator of channel c.  The reference
 // reduces its first lut_channels channels through a byte table
 // (csrc/rns_cuda.cu:69-96) and the rest with Barrett; the residue is unique,
 // so every channel here takes the 24-bit arithmetic reduction, which needs
 // no table loads (those would queue behind the output stores).
 template <int RCAP>
-__device__ __forceinline__ uint32_t reduce_acc(const Epi<RCAP> &e, int c, int32_t v) {
+__device__ __forceinline__ uint32_t reduce_acc(const IntConsts<RCAP> &e, int c, int32_t v) {
   return canon_fast(v, FastMod{e.m[c], e.m24[c], e.c16[c], e.bias[c], e.negm[c]});
 }
 
@@ -530,7 +728,7 @@ __device__ __forceinline__ uint32_t reduce_acc(const Epi<RCAP> &e, int c, int32_
 // so they accumulate in 32 bits; later digits in 64 bits.  x > P/2 maps to
 // x - P (P = P_{c_act}), the reference's signed correction.
 template <int RCAP>
-__device__ __forceinline__ int64_t garner_value(const Epi<RCAP> &e, const uint32_t (&r)[RCAP], int c_act) {
+__device__ __forceinline__ int64_t garner_value(const IntConsts<RCAP> &e, const uint32_t (&r)[RCAP], int c_act) {
   uint32_t d[RCAP];
   uint32_t x32 = 0;
   uint64_t x64 = 0;
@@ -581,7 +779,7 @@ __device__ __forceinline__ int64_t garner_value(const Epi<RCAP> &e, const uint32
 // 2^23 + 9 * 254^2 = 13,260,328 < 2^24: one mod_small gives d_c.  Every
 // multiply is 24-bit.
 template <int RCAP>
-__device__ __forceinline__ int64_t garner_from_sums(const Epi<RCAP> &e, const int32_t (&v)[RCAP], int c_act) {
+__device__ __forceinline__ int64_t garner_from_sums(const IntConsts<RCAP> &e, const int32_t (&v)[RCAP], int c_act) {
   uint32_t d[RCAP];
   uint32_t x32 = 0;
   uint64_t x64 = 0;
@@ -659,27 +857,16 @@ __device__ __forceinline__ ColScale col_scale(const Epi<RCAP> &e, int col, int n
   return cs;
 }
 
-// Writes one output element.  The float chain is
-// ((float)y * a_scale) * w_scale[col] + bias[col], each step rounded to
+// Writes one float output element: ((float)y * a_scale) * w_scale[col] +
+// bias[col] from f = (float)y, each step rounded to
 // nearest even with no contraction: the op order of rns_linear.py:272-275.
 // The operators are written here, under the pragma, on purpose: HIP's
 // __fmul_rn / __fadd_rn are plain operators compiled with contraction on
 // in their own header, and after inlining the multiply and the add would
 // fuse into an FMA (one rounding instead of two).
-// Int64 outputs are written with non-temporal stores: the kernel never
-// reads them back, and streaming them past the L2 keeps the A and weight
-// lines the other tiles still read (C2 M=256 8.98 -> 8.72 us, C5 M=2048
-// about 1 % faster, measured A/B on one box).
-template <int RCAP, int OUT>
-__device__ __forceinline__ void store_value(const Epi<RCAP> &e, int64_t y, int64_t idx, ColScale cs) {
+template <int RCAP>
+__device__ __forceinline__ void store_float(const Epi<RCAP> &e, float f, int64_t idx, ColScale cs) {
 #pragma clang fp contract(off)
-  if (OUT == kOutInt64 || (OUT == kOutAny && e.out_dtype == RNSMX_INT64)) {
-    __builtin_nontemporal_store(y, &as_global<int64_t>(e.out)[idx]);
-    return;
-  }
-  // with up to 4 channels |y| <= P/2 < 2^31: the 32-bit conversion rounds
-  // the same integer the same way, in one instruction
-  float f = RCAP <= 4 ? static_cast<float>(static_cast<int32_t>(y)) : __ll2float_rn(y);
   f = f * e.a_scale;
   f = f * cs.w;
   if (e.bias_ptr != nullptr) f = f + cs.b;
@@ -692,23 +879,51 @@ __device__ __forceinline__ void store_value(const Epi<RCAP> &e, int64_t y, int64
   }
 }
 
-// Reduction + reconstruction + store of one element from its channel sums.
-// FAST: every channel active (the common case), so the channel loop and
-// Garner run with no per-element branch.
+// Writes one output element.
+// Int64 outputs are written with non-temporal stores: the kernel never
+// reads them back, and streaming them past the L2 keeps the A and weight
+// lines the other tiles still read (C2 M=256 8.98 -> 8.72 us, C5 M=2048
+// about 1 % faster, measured A/B on one box).
+template <int RCAP, int OUT>
+__device__ __forceinline__ void store_value(const Epi<RCAP> &e, int64_t y, int64_t idx, ColScale cs) {
+  if (OUT == kOutInt64 || (OUT == kOutAny && e.out_dtype == RNSMX_INT64)) {
+    __builtin_nontemporal_store(y, &as_global<int64_t>(e.out)[idx]);
+    return;
+  }
+  // with up to 4 channels |y| <= P/2 < 2^31: the 32-bit conversion rounds
+  // the same integer the same way, in one instruction
+  store_float<RCAP>(e, RCAP <= 4 ? static_cast<float>(static_cast<int32_t>(y)) : __ll2float_rn(y), idx, cs);
+}
+
+// Reconstruction + store of one element from its channel sums.
+// FAST: every channel active (the common case), so the integer path's channel
+// loop runs with no per-element branch; by fractions every prefix runs the
+// same code.
 // idx = row * out_ld + col, the element's offset in the output; cs the
 // column's float-epilogue factors (col_scale).
 template <int RCAP, bool FAST, int OUT>
-__device__ __forceinline__ void finish_element(KArgs<RCAP> &g, const Epi<RCAP> &e, int c_act,
-                                               const int32_t (&v)[RCAP], int64_t idx, ColScale cs) {
-  const int64_t y = garner_from_sums<RCAP>(e, v, FAST ? RCAP : c_act);
-  store_value<RCAP, OUT>(e, y, idx, cs);
+__device__ __forceinline__ void finish_element(const Epi<RCAP> &e, int c_act, const int32_t (&v)[RCAP], int64_t idx,
+                                               ColScale cs) {
+  if constexpr (kFrac<RCAP>) {
+    const double t = frac_sum<RCAP>(e, v);
+    if constexpr (OUT == kOutInt64) {
+      store_value<RCAP, OUT>(e, frac_int<RCAP>(t), idx, cs);
+    } else {
+      // the same integer rounded to float the same way
+      const float f = RCAP <= 4 ? static_cast<float>(static_cast<int32_t>(__builtin_bit_cast(uint64_t, t)))
+                                : static_cast<float>(t - kRoundMagic);
+      store_float<RCAP>(e, f, idx, cs);
+    }
+  } else {
+    store_value<RCAP, OUT>(e, garner_from_sums<RCAP>(e.ic, v, FAST ? RCAP : c_act), idx, cs);
+  }
 }
 
 // Calls f(FAST, OUT) with the epilogue variant for this call: a uniform
 // branch taken once per workgroup instead of once per element.
 template <int RCAP, typename F>
 __device__ __forceinline__ void with_epilogue(const Epi<RCAP> &e, int c_act, F &&f) {
-  if (c_act == RCAP) {
+  if (kFrac<RCAP> || c_act == RCAP) {
     if (e.out_dtype == RNSMX_INT64)
       f(std::true_type{}, std::integral_constant<int, kOutInt64>{});
     else
@@ -767,7 +982,8 @@ __device__ __forceinline__ void register_epilogue(KArgs<RCAP> &g, const Epi<RCAP
   const int64_t idx0 = static_cast<int64_t>(r0 + 4 * (lane >> 4)) * e.out_ld + c0 + (lane & 15);
   const bool interior = r0 + 16 * MI <= m_lim && c0 + 16 * NJ <= n_lim;
   // int64 interior tiles with 16-byte aligned rows: two columns per store
-  const bool pairs = interior && e.out_dtype == RNSMX_INT64 && c_act == RCAP && (e.out_ld & 1) == 0 &&
+  const bool pairs = interior && e.out_dtype == RNSMX_INT64 && (kFrac<RCAP> || c_act == RCAP) &&
+                     (e.out_ld & 1) == 0 &&
                      (reinterpret_cast<uintptr_t>(e.out) & 15) == 0 && (c0 & 1) == 0;
   if (pairs) {
     const int64_t pidx0 = static_cast<int64_t>(r0 + 4 * (lane >> 4)) * e.out_ld + c0 + (lane & 14);
@@ -782,7 +998,10 @@ __device__ __forceinline__ void register_epilogue(KArgs<RCAP> &g, const Epi<RCAP
           constexpr int t = decltype(T)::value;
           int32_t v[RCAP];
           static_for<RCAP>([&](auto C) { v[decltype(C)::value] = acc[decltype(C)::value][i][j][t]; });
-          y[t] = garner_from_sums<RCAP>(e, v, RCAP);
+          if constexpr (kFrac<RCAP>)
+            y[t] = frac_int<RCAP>(frac_sum<RCAP>(e, v));
+          else
+            y[t] = garner_from_sums<RCAP>(e.ic, v, RCAP);
         });
         store_int64_pairs(y, as_global<int64_t>(e.out) + pidx0 + roff + j * 16, e.out_ld);
       });
@@ -806,7 +1025,7 @@ __device__ __forceinline__ void register_epilogue(KArgs<RCAP> &g, const Epi<RCAP
           if (decltype(INTERIOR)::value || (row < m_lim && col < n_lim)) {
             int32_t v[RCAP];
             static_for<RCAP>([&](auto C) { v[decltype(C)::value] = acc[decltype(C)::value][i][j][t]; });
-            finish_element<RCAP, decltype(FAST)::value, decltype(OUT)::value>(g, e, c_act, v,
+            finish_element<RCAP, decltype(FAST)::value, decltype(OUT)::value>(e, c_act, v,
                                                                               idx0 + roff + j * 16, cs[j]);
           }
         });
@@ -1021,6 +1240,7 @@ __device__ __forceinline__ bool split_exchange(KArgs<RCAP> &g, const Epi<RCAP> &
   constexpr int CH = MI * NJ * XW;  // 1 KB blocks per wave and split
   const int lane = threadIdx.x & 63;
   const int S = g.splits;
+  const IntConsts<RCAP> ic = int_consts<RCAP>(g, e, 0);
   int8_t *base = g.xchg + slot * S * CH * 1024 + lane * 4;
   auto block = [&](int s, int i, int j, int wd) {
     return base + (static_cast<int64_t>(s) * CH + (i * NJ + j) * XW + wd) * 1024;
@@ -1038,7 +1258,7 @@ __device__ __forceinline__ bool split_exchange(KArgs<RCAP> &g, const Epi<RCAP> &
           uint32_t packed = 0;
           static_for<4>([&](auto B) {
             constexpr int c = 4 * wd + decltype(B)::value;
-            if constexpr (c < RCAP) packed |= (reduce_acc<RCAP>(e, c, acc[c][i][j][t]) & 0xFFu) << (8 * (c % 4));
+            if constexpr (c < RCAP) packed |= (reduce_acc<RCAP>(ic, c, acc[c][i][j][t]) & 0xFFu) << (8 * (c % 4));
           });
           w[t] = static_cast<int32_t>(packed);
         });
@@ -1255,10 +1475,13 @@ __device__ __forceinline__ void stream_main(KArgs<RCAP> &g, const int c_act) {
   };
   auto mfma_chunk = [&]() { mfma_part(std::integral_constant<int, 0>{}, std::integral_constant<int, U>{}); };
 
+  Epi<RCAP> e;
+  if constexpr (kFrac<RCAP>) {
+    if (c_act != g.mods.channels) prefix_frac<RCAP>(g, e, c_act);
+  }
   // first chunk in flight before the epilogue constants are waited for
   load_chunk(wave * U);
-  Epi<RCAP> e;
-  load_epi<RCAP>(g, e, c_act);
+  load_epi<RCAP, false>(g, e, c_act);
   pin_epi<RCAP>(e);
   int m_lim = g.m, n_lim = g.n;
   pin_sgpr(m_lim);
@@ -1331,7 +1554,7 @@ __device__ __forceinline__ void stream_main(KArgs<RCAP> &g, const int c_act) {
               static_for<RCAP>([&](auto C) { v[decltype(C)::value] = acc[decltype(C)::value][i][j][t]; });
               // the row step is uniform: only idx0 is per lane
               const int64_t idx = idx0 + (i * 16 + t) * e.out_ld + j * 16;
-              finish_element<RCAP, decltype(FAST)::value, decltype(OUT)::value>(g, e, c_act, v, idx, cs[j]);
+              finish_element<RCAP, decltype(FAST)::value, decltype(OUT)::value>(e, c_act, v, idx, cs[j]);
             }
           });
         });
@@ -1369,7 +1592,7 @@ __device__ __forceinline__ void stream_main(KArgs<RCAP> &g, const int c_act) {
         int32_t v[RCAP];
         static_for<RCAP>([&](auto C) { v[decltype(C)::value] = sacc[decltype(C)::value * TILE + x]; });
         finish_element<RCAP, decltype(FAST)::value, decltype(OUT)::value>(
-            g, e, c_act, v, static_cast<int64_t>(m0 + x / BN) * e.out_ld + n0 + x % BN, cs1);
+            e, c_act, v, static_cast<int64_t>(m0 + x / BN) * e.out_ld + n0 + x % BN, cs1);
       }
     });
     return;
@@ -1391,7 +1614,7 @@ __device__ __forceinline__ void stream_main(KArgs<RCAP> &g, const int c_act) {
           int32_t v[RCAP];
           static_for<RCAP>([&](auto C) { v[decltype(C)::value] = sv[decltype(C)::value][v4]; });
           finish_element<RCAP, decltype(FAST)::value, decltype(OUT)::value>(
-              g, e, c_act, v, static_cast<int64_t>(m0 + row) * e.out_ld + n0 + col + v4, cs[v4]);
+              e, c_act, v, static_cast<int64_t>(m0 + row) * e.out_ld + n0 + col + v4, cs[v4]);
         }
       });
     }
@@ -1536,10 +1759,11 @@ __global__ __launch_bounds__(256) void rows_packed_kernel(const GemmArgsK<RCAP> 
   constexpr std::integral_constant<int, U / 2> h1{};
   constexpr std::integral_constant<int, U> h2{};
   int q = wave * U;
+  Epi<RCAP> e;
+  if (c_act != g.mods.channels) prefix_frac<RCAP>(g, e, c_act);
   load_part(q, h0, h1);
   load_part(q, h1, h2);
-  Epi<RCAP> e;
-  load_epi<RCAP>(g, e, c_act);
+  load_epi<RCAP, false>(g, e, c_act);
   pin_epi<RCAP>(e);
   for (int i = threadIdx.x; i < NBLK * 256; i += nthreads) (&sums[0][0][0])[i] = 0;
   if (q < nk) {
@@ -1573,7 +1797,7 @@ __global__ __launch_bounds__(256) void rows_packed_kernel(const GemmArgsK<RCAP> 
       int32_t v[RCAP];
       static_for<RCAP>([&](auto C) { v[decltype(C)::value] = sums[b][row0 + decltype(C)::value][j]; });
       finish_element<RCAP, decltype(FAST)::value, decltype(OUT)::value>(
-          g, e, c_act, v, static_cast<int64_t>(token) * e.out_ld + col, col_scale<RCAP>(e, col, n_lim));
+          e, c_act, v, static_cast<int64_t>(token) * e.out_ld + col, col_scale<RCAP>(e, col, n_lim));
     }
   });
 }
@@ -1938,16 +2162,6 @@ __device__ __forceinline__ void lds_body(KArgs<RCAP> &g, int8_t *smem, const int
     fb[c][j] = *reinterpret_cast<const i32x4 *>(rbase + st * STAGE + (AF + c * 4 + wn * NJ + j) * 1024);
   };
   i32x4 acc[RCAP][MI][NJ];
-  static_for<RCAP>([&](auto C) {
-    static_for<MI>([&](auto I) {
-      static_for<NJ>([&](auto J) {
-        if constexpr (decltype(C)::value < CA)
-          acc[C][I][J] = acc_zero();
-        else
-          acc[C][I][J] = i32x4{0, 0, 0, 0};
-      });
-    });
-  });
   // one K step k at stage h: wait until step k + 1 landed (own loads, then
   // everyone's, which also frees the stage of k - 1 and, at odd k with the
   // LDS reads of this step drained first, the A region of stage k), refill
@@ -2017,6 +2231,18 @@ __device__ __forceinline__ void lds_body(KArgs<RCAP> &g, int8_t *smem, const int
   const int rw0 = m0 + wm * (MI * 16), cw0 = n0 + wn * (NJ * 16);
   ColScale cs[NJ];
   static_for<NJ>([&](auto J) { cs[J] = col_scale<RCAP>(e, cw0 + decltype(J)::value * 16 + (lane & 15), n_lim); });
+  // after the constants of the epilogue: deriving those of a shorter prefix
+  // (prefix_frac) needs registers that the accumulators would hold
+  static_for<RCAP>([&](auto C) {
+    static_for<MI>([&](auto I) {
+      static_for<NJ>([&](auto J) {
+        if constexpr (decltype(C)::value < CA)
+          acc[C][I][J] = acc_zero();
+        else
+          acc[C][I][J] = i32x4{0, 0, 0, 0};
+      });
+    });
+  });
   // step 0 landed: at most the B loads of steps 1, 2 and the second A pair
   // (or fewer, when column factors were loaded after them) in flight
   wait_vmcnt<2 * BU + AU2>();
@@ -2182,16 +2408,6 @@ __device__ __forceinline__ void lds_wide_body(KArgs<RCAP> &g, int8_t *smem, cons
   };
 
   i32x4 acc[RCAP][MI][NJ];
-  static_for<RCAP>([&](auto C) {
-    static_for<MI>([&](auto I) {
-      static_for<NJ>([&](auto J) {
-        if constexpr (decltype(C)::value < CA)
-          acc[C][I][J] = acc_zero();
-        else
-          acc[C][I][J] = i32x4{0, 0, 0, 0};
-      });
-    });
-  });
 
   // one K step k at stage h: own loads of step k + 1 landed, then
   // everyone's (and everyone is done with step k - 1); this step's loads
@@ -2254,6 +2470,18 @@ __device__ __forceinline__ void lds_wide_body(KArgs<RCAP> &g, int8_t *smem, cons
   const int rw0 = m0 + wm * (MI * 16), cw0 = n0 + wn * (NJ * 16);
   ColScale cs[NJ];
   static_for<NJ>([&](auto J) { cs[J] = col_scale<RCAP>(e, cw0 + decltype(J)::value * 16 + (lane & 15), n_lim); });
+  // after the constants of the epilogue: deriving those of a shorter prefix
+  // (prefix_frac) needs registers that the accumulators would hold
+  static_for<RCAP>([&](auto C) {
+    static_for<MI>([&](auto I) {
+      static_for<NJ>([&](auto J) {
+        if constexpr (decltype(C)::value < CA)
+          acc[C][I][J] = acc_zero();
+        else
+          acc[C][I][J] = i32x4{0, 0, 0, 0};
+      });
+    });
+  });
   // step 0 landed (the column factors, when loaded, were issued after the
   // loads and are waited for too)
   wait_vmcnt<2 * BU>();
@@ -2485,9 +2713,11 @@ __device__ __forceinline__ void lds_planes_body(KArgs<RCAP> &g, int8_t *smem, co
   // factors 4 vector registers) through the loop, which the accumulators
   // leave no room for.  The scalar ones hit the constant cache (the
   // argument block was read at entry).
+  KArgs<RCAP> &late = args_from_here<RCAP>(g);
   Epi<RCAP> e;
-  load_epi<RCAP>(g, e, c_act);
-  const int m_lim = g.m, n_lim = g.n;
+  load_epi<RCAP>(late, e, c_act);
+  pin_epi<RCAP>(e);  // without it four accumulators are spilled inside the loop
+  const int m_lim = late.m, n_lim = late.n;
   if (wu.split >= 0 &&
       !split_exchange<RCAP, MI, NJ>(g, e, acc, static_cast<int64_t>(wu.split_tile) * NW + wave, wu.split))
     return;

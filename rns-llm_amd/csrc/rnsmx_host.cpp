@@ -1,4 +1,5 @@
 // Host-only part of the rnsmx C ABI: error text, moduli constants, LUT.
+#include <cmath>
 #include <cstring>
 
 #include "rnsmx_common.hpp"
@@ -32,6 +33,63 @@ static uint32_t inverse_mod(int64_t a, int64_t m) {
   for (int64_t x = 1; x < m; ++x)
     if ((r * x) % m == 1) return static_cast<uint32_t>(x);
   return m == 1 ? 0u : 0xFFFFFFFFu;
+}
+
+// Inverse of a modulo m, 0 < a < m <= 255 coprime, by Euclid's algorithm.
+static int inverse_euclid(int a, int m) {
+  int r0 = m, r1 = a, t0 = 0, t1 = 1;
+  while (r1 != 0) {
+    const int q = r0 / r1;
+    const int r = r0 - q * r1, t = t0 - q * t1;
+    r0 = r1;
+    r1 = r;
+    t0 = t1;
+    t1 = t;
+  }
+  return t0 < 0 ? t0 + m : t0;
+}
+
+static FracSet make_frac_set(const rnsmx_moduli_t &mods) {
+  FracSet s{};
+  const int channels = mods.channels;
+  if (channels < 1 || channels > 6) return s;
+  for (int p = 1; p <= channels; ++p) {
+    for (int c = 0; c < p; ++c) {
+      const int m = mods.moduli[c];
+      int rest = 1;  // P_p / m_c mod m_c
+      for (int j = 0; j < p; ++j)
+        if (j != c) rest = rest * (mods.moduli[j] % m) % m;
+      int k = inverse_euclid(rest, m);
+      if (2 * k > m) k -= m;
+      s.kprefix[p][c / 4] |= (static_cast<uint32_t>(k) & 0xFFu) << (8 * (c % 4));
+      if (p == channels) {
+        const double md = m, kd = k, s20 = 1048576.0, s40 = 1048576.0 * 1048576.0;
+        s.row0[c] = std::rint(kd / md * s20) / s20;
+        const double r1 = std::fma(-s.row0[c], md, kd);  // exact
+        s.rest1[c] = r1 / md;
+        s.row1[c] = std::rint(r1 / md * s40) / s40;
+        s.rest2[c] = std::fma(-s.row1[c], md, r1) / md;
+      }
+    }
+  }
+  const int64_t p = mods.prefix[channels];  // below 2^48
+  s.p = static_cast<double>(p);
+  s.half = static_cast<double>((p - 1) >> 1);
+  s.turn = (s.half + 0.25) / s.p;
+  return s;
+}
+
+const FracSet &frac_set(const rnsmx_moduli_t &mods) {
+  static thread_local int32_t channels = 0;
+  static thread_local int32_t moduli[RNSMX_MAX_CHANNELS] = {};
+  static thread_local FracSet set{};
+  const size_t bytes = sizeof(int32_t) * static_cast<size_t>(mods.channels);
+  if (mods.channels != channels || std::memcmp(moduli, mods.moduli, bytes) != 0) {
+    set = make_frac_set(mods);
+    std::memcpy(moduli, mods.moduli, bytes);
+    channels = mods.channels;
+  }
+  return set;
 }
 
 }  // namespace rnsmx

@@ -487,7 +487,7 @@ struct DecodeArgs {
 template <int RCAP>
 __global__ __launch_bounds__(256) void decode_garner_kernel(const DecodeArgs a) {
   const int R = a.mods.channels;
-  Epi<RCAP> k;
+  IntConsts<RCAP> k;
   fill_moduli<RCAP>(k, a.mods, R);
   for (int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < a.count;
        e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
