@@ -89,7 +89,11 @@ typedef struct rnsmx_moduli {
  * LDS-staged kernel with 256 x 96 tiles (same conditions as 3), 8 = the
  * LDS-staged kernel for residue-plane activations (int16 / int32 inputs,
  * and packed weights; 128 x 128 tiles, 4- or 6-channel capacity, K a
- * multiple of 256; mb, nb, ks ignored; splits and tail as for kind 3).
+ * multiple of 256; mb, nb, ks ignored; splits and tail as for kind 3), 9 and
+ * 10 = packed weights by byte products (int8 and int16 activations, K up to
+ * 65472): 9 reads the activations as they are (up to mb = 1, 2 or 4 fragments
+ * of 8 int16 or 16 int8 tokens, ks waves splitting K, never split), 10 runs
+ * tiles of 16*mb x 24*mb (mb 4 or 8), split as kind 3.
  * splits: workgroups splitting K per output tile (0 or 1 = none; up to 4
  * channels, 6 for kind 8, and for the stream kernel ks = 1): each reduces its partial
  * sums to residues, and the last to finish a tile reconstructs it.  tail:
@@ -296,11 +300,17 @@ int32_t rnsmx_matmul_residues_prepared(
  *
  * rnsmx_matmul_packed_fused: rnsmx_matmul_prepared_fused against a packed
  * weight, with the same arguments, results and errors, for 2 to 6
- * channels.  Channel c's weight residue is never stored: with
+ * channels.  int8 and int16 activations (K up to 65472) run by byte
+ * products: the exact sum of the products of the weight's and the
+ * activations' bytes, taken to the centered range of the active channels'
+ * product, which is what their residues reconstruct to.  Otherwise (int32
+ * activations, longer K, or a plan that asks for it) by channels: channel
+ * c's weight residue is never stored: with
  * d_c = 256 mod m_c, v = d_c hi + lo + 128 (mod m_c), so the kernels run
  * two MFMAs per channel (activation residues of d_c a against hi, of a
  * against lo) and add 128 sum_k a_k per row.  Accumulators: 2 K 128
- * max(floor(m/2)) + 255 < 2^31 (else RNSMX_ERANGE).  Plans: kind 1 (stream,
+ * max(floor(m/2)) + 255 < 2^31 (else RNSMX_ERANGE).  Plans: kinds 9 and 10
+ * (byte products) and, by channels, kind 1 (stream,
  * mb 1 or 2, nb 1, ks 1-4), 2 (MFMA, mb 2 or 4, nb 1) or 6 (channel rows,
  * mb 1, 2, 4 or 8 token blocks), never split, or 8 (the residue-plane LDS
  * kernel, K a multiple of 256, split as for the residue-plane entry); NULL
@@ -327,7 +337,8 @@ int32_t rnsmx_matmul_packed_fused(
     const rnsmx_plan_t *plan, void *workspace_dev, int64_t workspace_bytes,
     void *out_dev, void *stream);
 
-/* The plan rnsmx_matmul_packed_fused chooses by itself (host only). */
+/* The plan rnsmx_matmul_packed_fused chooses by itself for int32 activations
+ * (host only); int8 and int16 ones take byte products (kinds 9 and 10). */
 int32_t rnsmx_packed_plan(int64_t m, int64_t n, int64_t k, int32_t channels,
                           rnsmx_plan_t *out);
 

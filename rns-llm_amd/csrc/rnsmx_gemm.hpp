@@ -165,6 +165,8 @@ inline GemmArgsK<RCAP> compact_args(const GemmArgs &g) {
 // kMfma3: the MFMA kernel with three column waves (48*nb-column tiles).
 // kRows: packed weights at decode (rows_packed_kernel: MFMA rows are channels).
 // kLdsWide: the LDS-staged kernel with 256 x 96 tiles (lds_wide_kernel).
+// kBytesRows, kBytesLds: packed weights by byte products (rnsmx_bytes.hpp):
+// decode (mb fragments of tokens), tiles of 16 mb rows.
 enum GemmKind {
   kAuto = 0,
   kStream = 1,
@@ -174,7 +176,9 @@ enum GemmKind {
   kMfma3 = 5,
   kRows = 6,
   kLdsWide = 7,
-  kLdsPlanes = 8
+  kLdsPlanes = 8,
+  kBytesRows = 9,
+  kBytesLds = 10
 };
 
 // ks: waves splitting K (stream kernel) or ring depth, 0 = automatic (MFMA
@@ -218,6 +222,9 @@ RNSMX_GEMM_PARTS_DECL(3)
 RNSMX_GEMM_PARTS_DECL(4)
 RNSMX_GEMM_PARTS_DECL(6)
 RNSMX_GEMM_PARTS_DECL(10)
+// The byte-product kernels (rnsmx_bytes.hip), ab bytes per activation; false
+// when there is none for the choice.
+bool launch_bytes(const GemmArgs &g, int ab, const GemmChoice &c, hipStream_t st);
 
 // Kernel arguments read in place from the kernarg segment (constant address
 // space, scalar loads).  A by-value struct parameter used as an ordinary
@@ -2890,6 +2897,15 @@ inline GemmGrid gemm_grid(const GemmChoice &c, int64_t m, int64_t n) {
     r.tiles = cdiv(m, kLdsBM) * cdiv(n, bn);
     r.waves = 8;
     r.chunks = (kLdsBM / 16 / 4) * (bn / 16 / 2);
+  } else if (c.kind == kBytesRows) {
+    r.tiles = cdiv(n, 16);
+    r.waves = c.ks;
+    r.chunks = c.mb;
+  } else if (c.kind == kBytesLds) {
+    // 128 x 192 (8 waves of 64 x 48) or 64 x 96 (4 of 32 x 48); two words per element
+    r.tiles = cdiv(m, 16 * c.mb) * cdiv(n, 24 * c.mb);
+    r.waves = c.mb;
+    r.chunks = c.mb / 2 * 3 * 2;
   } else if (c.kind == kLdsPlanes) {
     r.tiles = cdiv(m, kPlBM) * cdiv(n, kPlBN);
     r.waves = 8;

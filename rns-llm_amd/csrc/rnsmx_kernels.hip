@@ -18,6 +18,7 @@
 #include <climits>
 #include <mutex>
 
+#include "rnsmx_bytes.hpp"
 #include "rnsmx_gemm.hpp"
 
 namespace rnsmx {
@@ -372,6 +373,56 @@ __global__ __launch_bounds__(256) void encode_token_rows_kernel(const TokenRowsA
   reinterpret_cast<uint32_t *>(e.out)[word] = packed;
 }
 
+// Activations for the byte-product tiles (rnsmx_bytes.hpp): int16 rows as
+// planes ah = a >> 8 and al = (a & 255) - 128 (int8 rows as they are),
+// [planes][rows][out_ld], K past cols as a = 0, and the row terms 128 sum_k a
+// as doubles after the planes; the row L1 norm too when asked.  One workgroup
+// per row, a thread per 16 values: 2 planes instead of the 12 (and 12 row
+// terms) of six channels, 512 rows of K = 4096 in 5 us instead of 19.
+template <typename T>
+__global__ __launch_bounds__(256) void bytes_planes_kernel(const EncodeArgs e) {
+  constexpr int AB = sizeof(T);
+  __shared__ int64_t sh[16];
+  const int64_t row = blockIdx.x;
+  const T *src = static_cast<const T *>(e.values) + row * e.cols;
+  const bool vec = e.cols % (16 / AB) == 0;
+  int64_t l1 = 0;
+  int32_t sum = 0;  // 16 values of at most 2^15 per pass, K below 2^16
+  for (int64_t k0 = static_cast<int64_t>(threadIdx.x) * 16; k0 < e.out_ld; k0 += static_cast<int64_t>(blockDim.x) * 16) {
+    int32_t v[16];
+    if (vec && k0 + 16 <= e.cols) {
+      load16<T>(src + k0, v);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) v[q] = (k0 + q < e.cols) ? static_cast<int32_t>(src[k0 + q]) : 0;
+    }
+    i32x4 hi, lo;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      uint32_t h = 0, l = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int32_t x = v[4 * d + q];
+        sum += x;
+        if (e.row_l1 != nullptr) l1 += x < 0 ? -x : x;
+        h |= (static_cast<uint32_t>(AB == 2 ? x >> 8 : x) & 0xFFu) << (8 * q);
+        l |= ((static_cast<uint32_t>(x) & 0xFFu) ^ 0x80u) << (8 * q);
+      }
+      hi[d] = static_cast<int32_t>(h);
+      lo[d] = static_cast<int32_t>(l);
+    }
+    *reinterpret_cast<i32x4 *>(e.out + row * e.out_ld + k0) = hi;
+    if constexpr (AB == 2) *reinterpret_cast<i32x4 *>(e.out + e.plane + row * e.out_ld + k0) = lo;
+  }
+  const int64_t total = block_sum_i64(sum, sh);
+  if (threadIdx.x == 0)
+    reinterpret_cast<double *>(e.out + AB * e.plane)[row] = 128.0 * static_cast<double>(total);
+  if (e.row_l1 != nullptr) {
+    l1 = block_sum_i64(l1, sh);
+    if (threadIdx.x == 0) e.row_l1[row] = l1;
+  }
+}
+
 // Packed weight preparation: int8/int16 [N][K] -> two byte planes in the
 // fragment-major order of encode_frag_kernel ([2][N16][nk][1024]): hi =
 // v >> 8 and lo = (v & 255) - 128, so v = 256 hi + lo + 128 with both bytes
@@ -580,7 +631,9 @@ static int rcap_for(int channels) {
   return 10;
 }
 
-static bool is_lds(int kind) { return kind == kLds || kind == kLdsWide || kind == kLdsPlanes; }
+static bool is_lds(int kind) {
+  return kind == kLds || kind == kLdsWide || kind == kLdsPlanes || kind == kBytesLds;
+}
 
 static int32_t check_launch(const char *what) {
   const hipError_t err = hipGetLastError();
@@ -897,6 +950,8 @@ static bool split_fits(const GemmChoice &c, const GemmArgs &g) {
     built = stream_splits(rcap, c.mb, c.nb) && c.ks == 1;
   else if (c.kind == kLdsPlanes)
     built = rcap == 4 || rcap == 6;
+  else if (c.kind == kBytesLds)
+    built = true;
   else if (is_lds(c.kind))
     built = rcap <= 4;
   else
@@ -912,7 +967,8 @@ static int64_t xchg_bytes(const GemmChoice &c, const GemmArgs &g) {
   if (splits <= 1) return 0;
   const GemmGrid gr = gemm_grid(c, g.m, g.n);
   const int64_t parted = gr.tiles - whole_tiles(c, gr.tiles);
-  const int words = (rcap_for(g.mods.channels) + 3) / 4;  // residue words per element (xchg_words)
+  // residue words per element (xchg_words); the byte products' own count holds theirs
+  const int words = c.kind == kBytesLds ? 1 : (rcap_for(g.mods.channels) + 3) / 4;
   return round_up(parted * gr.waves * splits * gr.chunks * words * 1024, 256);
 }
 
@@ -1029,7 +1085,7 @@ static int32_t launch_gemm(GemmArgs g, bool araw, const GemmChoice &c, uint32_t 
   const int64_t tiles = gemm_grid(c, g.m, g.n).tiles;
   g.split_from = static_cast<int32_t>(tiles);
   if (c.splits > 1) {
-    if (is_lds(c.kind) &&
+    if (is_lds(c.kind) && c.kind != kBytesLds &&
         !(c.kind == kLdsPlanes ? lds_planes_fits(g, araw, rcap) : lds_kernel_fits(g, araw, rcap))) {
       set_error("no GEMM kernel for kind %d, tile %d x %d, %d channels", c.kind, c.mb, c.nb, g.mods.channels);
       return RNSMX_EINVAL;
@@ -1038,6 +1094,13 @@ static int32_t launch_gemm(GemmArgs g, bool araw, const GemmChoice &c, uint32_t 
     if (g.splits > 1 && (tickets == nullptr || xchg == nullptr))
       return fail(RNSMX_EINVAL, "a K split needs the workspace's counters and exchange area");
     if (g.splits > 1) g.split_from = static_cast<int32_t>(whole_tiles(c, tiles));
+  }
+  if (c.kind == kBytesRows || c.kind == kBytesLds) {
+    if (!launch_bytes(g, araw ? 1 : 2, c, st)) {
+      set_error("no byte-product kernel for kind %d, tile %d", c.kind, c.mb);
+      return RNSMX_EINVAL;
+    }
+    return check_launch("gemm_bytes");
   }
   using PartFn = bool (*)(const GemmArgs &, bool, const GemmChoice &, hipStream_t);
 #define RNSMX_PARTS(R)                                                                      \
@@ -1156,9 +1219,68 @@ static GemmChoice packed_auto(const GemmArgs &g) {
   return c;
 }
 
-static int32_t packed_plan_from(const rnsmx_plan_t *plan, const GemmArgs &g, GemmChoice &c) {
+// Byte products (rnsmx_bytes.hpp) for int8 (ab = 1) and int16 (ab = 2)
+// activations, K within the int32 sums.
+static bool bytes_fit(const GemmArgs &g) { return g.kp <= kBytesMaxKp; }
+
+// Kernel, tile and split for byte products, from a sweep on MI355X (int16, K
+// 768-4096, N 768-12288, M 16-4096; us per call, planes launch included).
+// Rows: up to two fragments of tokens (K=4096 N=12288 M=4 20.3, M=16 30-32
+// against 30.8 on tiles), four where the weight is small (16 M values: M=24
+// 21.3 against 24.2, M=32 24.6 against 23.8; K=4096 N=12288 M=32 52 against
+// 31: every workgroup of 16 columns reads all the activations).
+// Tiles: 64 x 96 run two workgroups per CU, 128 x 192 one.  Cost of a round
+// over nk K steps (us): up to 256 small tiles 5.4 + 0.385 nk, up to 512 10 +
+// 0.58 nk, up to 256 large ones 12.5 + 0.96 nk; the sum picks the faster tile
+// at all but three of the 90 shapes (those within 8 %): N=12288 K=4096 M=256
+// 58.8 small against 70.3, M=512 87 large against 107.
+// Split: where the tiles and their splits fit one round of 256, each keeping
+// 16 K steps (N=12288 K=4096 M=64, 128 small tiles, 31.9 in two halves against
+// 36.9; N=4096 M=64 23.8 in four against 27; at K = 1024 a split loses, 15.5
+// against 14.0).
+static GemmChoice bytes_auto(const GemmArgs &g, int ab) {
+  const int tpf = 16 / ab;
+  const int nk = g.kp / 64;
+  const bool small_weight = static_cast<int64_t>(g.n) * g.kp <= (int64_t{1} << 24);
+  if (g.m <= (small_weight ? 4 : 2) * tpf) {
+    const int nf = g.m <= tpf ? 1 : g.m <= 2 * tpf ? 2 : 4;
+    const int per = 8 + 4 * ab * nf, u = per <= 16 ? 8 : per <= 24 ? 4 : 2;  // bytes_rows_u
+    return GemmChoice{kBytesRows, nf, 1, std::min(4, std::max(1, (nk + u - 1) / u)), 1, 0};
+  }
+  GemmChoice c{kBytesLds, 4, 0, 0, 1, 0}, large{kBytesLds, 8, 0, 0, 1, 0};
+  const int64_t ts = gemm_grid(c, g.m, g.n).tiles, tl = gemm_grid(large, g.m, g.n).tiles;
+  const double half_round = 5.4 + 0.385 * nk, round = 10 + 0.58 * nk;
+  const int64_t rest = ts % 512;
+  const double cost_s = static_cast<double>(ts / 512) * round + (rest == 0 ? 0 : rest <= 256 ? half_round : round);
+  const double cost_l = static_cast<double>((tl + 255) / 256) * (12.5 + 0.96 * nk);
+  if (cost_l < cost_s) c = large;
+  const int64_t tiles = std::min(ts, c.mb == 8 ? tl : ts);
+  while (2 * c.splits * tiles <= 256 && nk / (2 * c.splits) >= 16 && c.splits < 4) c.splits *= 2;
+  if (c.splits > 1 && !split_fits(c, g)) c.splits = 1;
+  return c;
+}
+
+// a_dtype: the activations' type (-1: not known yet, any plan they could take).
+static int32_t packed_plan_from(const rnsmx_plan_t *plan, const GemmArgs &g, GemmChoice &c, int32_t a_dtype = -1) {
   if (plan == nullptr || plan->kind == kAuto) {
-    c = packed_auto(g);
+    if ((a_dtype == RNSMX_INT8 || a_dtype == RNSMX_INT16) && bytes_fit(g))
+      c = bytes_auto(g, a_dtype == RNSMX_INT8 ? 1 : 2);
+    else
+      c = packed_auto(g);
+    return RNSMX_OK;
+  }
+  if (plan->kind == kBytesRows || plan->kind == kBytesLds) {
+    if (a_dtype == RNSMX_INT32 || !bytes_fit(g))
+      return fail(RNSMX_EINVAL, "byte-product plans take int8 or int16 activations and K up to 65472");
+    c = GemmChoice{plan->kind, plan->mb, 1, plan->ks, std::max(1, plan->splits), plan->tail != 0};
+    if (c.kind == kBytesRows) {
+      const int tokens = plan->mb * (a_dtype == RNSMX_INT8 ? 16 : 8);
+      if ((c.mb != 1 && c.mb != 2 && c.mb != 4) || c.ks < 1 || c.ks > 4 || c.splits > 1 || c.tail ||
+          (a_dtype >= 0 && g.m > tokens))
+        return fail(RNSMX_EINVAL, "byte-product rows: 1, 2 or 4 fragments that hold every token, 1-4 waves, no split");
+    } else if ((c.mb != 4 && c.mb != 8) || (c.splits > 1 && !split_fits(c, g))) {
+      return fail(RNSMX_EINVAL, "byte-product tiles: mb 4 or 8, splits within the counters");
+    }
     return RNSMX_OK;
   }
   const bool stream = plan->kind == kStream && (plan->mb == 1 || plan->mb == 2) && plan->nb == 1;
@@ -1603,7 +1725,9 @@ static PreparedLayout packed_layout(int64_t m, int64_t kp, int32_t channels, int
   PreparedLayout l{};
   l.a_res = kTicketBytes;
   // per-channel planes, or (up to 8 tokens) two blocks of channel-row fragments
-  const int64_t planes = 2 * channels * m * kp + 4 * channels * packed_corr_ld(m);
+  // (from 2 channels on this also holds the byte planes and their row terms)
+  const int64_t planes = std::max(2 * channels * m * kp + 4 * channels * packed_corr_ld(m),
+                                  2 * m * round_up(kp, 128) + 8 * packed_corr_ld(m));
   const int64_t rows = m <= kRowsMaxBlocks * 4 ? int64_t{kRowsMaxBlocks} * 2 * kp * 16 : 0;
   l.row_l1 = l.a_res + round_up(std::max(planes, rows), 256);
   l.xchg = l.row_l1 + round_up(8 * (m + 1), 256);  // the norms, then their maximum
@@ -1676,7 +1800,8 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   GemmArgs g = plan_args(m, n, k, R, araw);
   g.mods = *mods;
   GemmChoice c{};
-  if (int32_t rc = packed ? packed_plan_from(plan, g, c) : plan_from(plan, g, araw, true, c)) return rc;
+  if (int32_t rc = packed ? packed_plan_from(plan, g, c, a_dtype) : plan_from(plan, g, araw, true, c)) return rc;
+  const bool bytes = c.kind == kBytesRows || c.kind == kBytesLds;
   const PreparedLayout l = packed ? packed_layout(m, kp, R, xchg_bytes(c, g))
                                   : prepared_layout(araw, m, kp, R, xchg_bytes(c, g));
   if (workspace_bytes < l.total) {
@@ -1705,7 +1830,40 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   e.absmax = nullptr;
   e.mods = *mods;
   const bool rows = packed && c.kind == kRows;
-  if (rows) {
+  const int ab = a_dtype == RNSMX_INT8 ? 1 : 2;  // bytes per activation (byte products)
+  if (c.kind == kBytesRows) {
+    // rows read as they are; rows that are not 16-byte aligned are copied
+    // to padded ones first
+    g.a = static_cast<const int8_t *>(a_dev);
+    g.a_ld = g.a_k = k;
+    if (static_cast<int64_t>(k) * ab % 16 != 0) {
+      const int64_t total = static_cast<int64_t>(m) * kp * ab;
+      hipLaunchKernelGGL(pad_rows_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, g.a,
+                         static_cast<int64_t>(m), static_cast<int64_t>(k) * ab, kp * ab, total, a_res);
+      if (int32_t rc = check_launch("pad_rows")) return rc;
+      g.a = a_res;
+      g.a_ld = kp;
+      g.a_k = static_cast<int32_t>(kp);
+    }
+    if (min_ch != 0) {  // the row norms of the adaptive bound
+      EncodeArgs l1 = e;
+      l1.out = nullptr;
+      if (int32_t rc = launch_encode_rows(a_dtype, l1, st)) return rc;
+    }
+  } else if (c.kind == kBytesLds) {
+    g.a = a_res;
+    g.a_ld = round_up(kp, 128);  // whole pairs of K steps
+    g.a_cs = g.a_ld * m;
+    EncodeArgs planes = e;
+    planes.out_ld = g.a_ld;
+    planes.plane = g.a_cs;
+    const unsigned threads = static_cast<unsigned>(std::min<int64_t>(256, (g.a_ld / 16 + 63) / 64 * 64));
+    if (ab == 1)
+      hipLaunchKernelGGL(bytes_planes_kernel<int8_t>, dim3(static_cast<unsigned>(m)), dim3(threads), 0, st, planes);
+    else
+      hipLaunchKernelGGL(bytes_planes_kernel<int16_t>, dim3(static_cast<unsigned>(m)), dim3(threads), 0, st, planes);
+    if (int32_t rc = check_launch("bytes_planes")) return rc;
+  } else if (rows) {
     TokenRowsArgs t{};
     t.values = a_dev;
     t.m = m;
@@ -1737,7 +1895,9 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
     if (int32_t rc = launch_encode_rows(a_dtype, e, st)) return rc;
   }
 
-  if (araw) {
+  if (bytes) {
+    // set above
+  } else if (araw) {
     g.a = static_cast<const int8_t *>(a_dev);
     g.a_cs = 0;
   } else {
@@ -1759,7 +1919,7 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   g.a_scale = epilogue ? epilogue->a_scale_dev : nullptr;
   g.w_scale = epilogue ? epilogue->w_scale_dev : nullptr;
   g.bias = epilogue ? epilogue->bias_dev : nullptr;
-  return launch_gemm(g, araw, c, reinterpret_cast<uint32_t *>(ws), ws + l.xchg, st, packed);
+  return launch_gemm(g, bytes ? ab == 1 : araw, c, reinterpret_cast<uint32_t *>(ws), ws + l.xchg, st, packed);
 }
 
 int64_t rnsmx_packed_workspace_bytes(int64_t m, int64_t k, int64_t n, int32_t channels,
@@ -1771,7 +1931,10 @@ int64_t rnsmx_packed_workspace_bytes(int64_t m, int64_t k, int64_t n, int32_t ch
                                false);
   GemmChoice c{};
   if (packed_plan_from(plan, g, c) != RNSMX_OK) return -1;
-  return packed_layout(m, g.kp, channels, xchg_bytes(c, g)).total;
+  int64_t xchg = xchg_bytes(c, g);
+  if ((plan == nullptr || plan->kind == kAuto) && bytes_fit(g))  // whatever the activations' type
+    for (int ab = 1; ab <= 2; ++ab) xchg = std::max(xchg, xchg_bytes(bytes_auto(g, ab), g));
+  return packed_layout(m, g.kp, channels, xchg).total;
 }
 
 int32_t rnsmx_matmul_prepared_fused(const void *a_dev, int32_t a_dtype, int32_t m, int32_t k, int32_t n,
