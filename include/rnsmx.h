@@ -236,6 +236,25 @@ int32_t rnsmx_matmul_prepared_fused(
     const rnsmx_plan_t *plan, void *workspace_dev, int64_t workspace_bytes,
     void *out_dev, void *stream);
 
+/*
+ * Both operands plain integers, used once: a_dev [M][K] and b_dev [K][N], both
+ * int8, int16 or int32 (row-major) -> exact out_dev [M][N] int64.  Encodes B
+ * straight into the fragment-major order of rnsmx_prepare_weight in the
+ * workspace and runs the prepared-weight product; the workspace may hold
+ * anything before the call (rnsmx_wide_workspace_bytes) and its counters are
+ * zero after it.
+ * Replaces the chain encode_centered (both operands) -> matmul_centered_fused
+ * of CudaRNSBackend.matmul_wide (cuda_backend.py:733-799).
+ */
+int64_t rnsmx_wide_workspace_bytes(int64_t m, int64_t k, int64_t n,
+                                   int32_t channels);
+
+int32_t rnsmx_matmul_wide(const void *a_dev, const void *b_dev, int32_t dtype,
+                          int32_t m, int32_t k, int32_t n,
+                          const rnsmx_moduli_t *mods, void *workspace_dev,
+                          int64_t workspace_bytes, int64_t *out_dev,
+                          void *stream);
+
 /* Bytes of the static scratch of rnsmx_matmul_prepared_fused_noalloc (16 MiB
  * per GPU, held until the process ends). */
 #define RNSMX_NOALLOC_SCRATCH_BYTES (16 << 20)

@@ -93,6 +93,30 @@ __device__ __forceinline__ int32_t centered_i32(int32_t v, uint32_t m, uint32_t 
                       : static_cast<int32_t>(r);
 }
 
+// Centered residues of small integers (|v| <= 2^15) in float: r = v - m floor(v
+// / m + turn) with turn = (h + 1/4) / m, h = (m - 1) >> 1, so r lies in [-h, m -
+// 1 - h] = the centered range (m / 2 itself for an even m).  v / m + turn is at
+// least 1 / (4 m) from an integer and misses by less than |v| / m * 2^-22, so
+// the floor is right; the fma on v + 1.5 * 2^23 is exact and leaves r in the low
+// byte.  Three instructions per value and modulus (centered_i32: about twelve).
+struct SmallMod {
+  float inv, turn, m;
+};
+__device__ __forceinline__ SmallMod small_mod_of(uint32_t m) {
+  const float f = static_cast<float>(m);
+  return SmallMod{1.0f / f, (static_cast<float>((m - 1) >> 1) + 0.25f) / f, f};
+}
+constexpr float kByteMagic = 12582912.0f;  // 1.5 * 2^23
+__device__ __forceinline__ uint32_t centered_byte(float v, const SmallMod &s) {
+  const float q = __builtin_floorf(__builtin_fmaf(v, s.inv, s.turn));
+  return __float_as_uint(__builtin_fmaf(-q, s.m, v + kByteMagic));  // the byte is the low one
+}
+// The low bytes of four words.
+__device__ __forceinline__ uint32_t pack_low_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  const uint32_t ab = __builtin_amdgcn_perm(b, a, 0x0c0c0400u), cd = __builtin_amdgcn_perm(d, c, 0x0c0c0400u);
+  return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
+}
+
 __device__ __forceinline__ uint32_t byte_of(uint32_t w, int t) {
   return (w >> (8 * t)) & 0xFFu;
 }

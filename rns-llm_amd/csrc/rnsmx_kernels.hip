@@ -274,6 +274,68 @@ __global__ __launch_bounds__(256) void encode_frag_kernel(const EncodeArgs e) {
   }
 }
 
+// The same from a weight stored [K][N] (rows of e.rows columns, e.cols of
+// them): a workgroup takes one K step (64 rows) of 64 columns through LDS, so
+// the rows are read as whole segments, and each wave writes the fragment of 16
+// columns for every channel.  Also clears the first `ntickets` split counters.
+// One pass over the plain integers in place of encoding them to [R][K][N] and
+// repacking that (2048 x 2048 int8, 4 channels: 25 us in two launches).
+template <typename T>
+__global__ __launch_bounds__(256) void encode_frag_kn_kernel(const EncodeArgs e, uint32_t *tickets, int64_t ntickets) {
+  constexpr int kRow = 64 + 4 / sizeof(T);  // one bank of padding
+  __shared__ T tile[64 * kRow];
+  for (int64_t q = (static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x; q < ntickets;
+       q += static_cast<int64_t>(gridDim.x) * gridDim.y * 256)
+    tickets[q] = 0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 64, ks = blockIdx.y, n = e.rows;
+  const T *src = static_cast<const T *>(e.values);
+  constexpr int V = 16 / sizeof(T);  // values per load
+  static_for<64 * 64 / V / 256>([&](auto U) {
+    const int q = decltype(U)::value * 256 + threadIdx.x;
+    const int r = q / (64 / V), c = q % (64 / V) * V;
+    const int64_t k = ks * 64 + r, col = n0 + c;
+    T v[V];
+    if (k < e.cols && col + V <= n) {
+      __builtin_memcpy(v, src + k * n + col, 16);
+    } else {
+      static_for<V>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        v[i] = k < e.cols && col + i < n ? src[k * n + col + i] : static_cast<T>(0);
+      });
+    }
+    __builtin_memcpy(&tile[r * kRow + c], v, 16);
+  });
+  __syncthreads();
+  const int64_t jb = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+  if (jb * 16 >= n) return;
+  const T *mine = tile + (lane >> 4) * 16 * kRow + wave * 16 + (lane & 15);
+  int8_t *dst = e.out + (jb * (e.out_ld / 64) + ks) * 1024 + lane * 16;
+  int32_t v[16];
+  static_for<16>([&](auto Q) { v[decltype(Q)::value] = static_cast<int32_t>(mine[decltype(Q)::value * kRow]); });
+  for (int c = 0; c < e.mods.channels; ++c) {
+    const uint32_t m = static_cast<uint32_t>(e.mods.moduli[c]);
+    i32x4 w;
+    if constexpr (sizeof(T) <= 2) {
+      const SmallMod s = small_mod_of(m);
+      static_for<4>([&](auto D) {
+        constexpr int d = 4 * decltype(D)::value;
+        w[decltype(D)::value] = static_cast<int32_t>(pack_low_bytes(
+            centered_byte(static_cast<float>(v[d]), s), centered_byte(static_cast<float>(v[d + 1]), s),
+            centered_byte(static_cast<float>(v[d + 2]), s), centered_byte(static_cast<float>(v[d + 3]), s)));
+      });
+    } else {
+      const uint32_t magic = e.mods.magic[c], c31 = e.mods.c31[c];
+      static_for<4>([&](auto D) {
+        constexpr int d = 4 * decltype(D)::value;
+        auto byte = [&](int i) { return static_cast<uint32_t>(centered_i32(v[i], m, magic, c31)); };
+        w[decltype(D)::value] = static_cast<int32_t>(pack_low_bytes(byte(d), byte(d + 1), byte(d + 2), byte(d + 3)));
+      });
+    }
+    *reinterpret_cast<i32x4 *>(dst + c * e.plane) = w;
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ void load4(const T *p, int32_t (&v)[4]) {
   if constexpr (sizeof(T) == 1) {
@@ -595,14 +657,25 @@ __global__ __launch_bounds__(256) void transpose_frag_kernel(const int8_t *__res
   }
 }
 
-// src [R][rows][K] -> dst [R][rows][ld], zero in [K, ld).
-__global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t *__restrict__ src, int64_t rows,
-                                                       int64_t k, int64_t ld, int64_t total,
-                                                       int8_t *__restrict__ dst) {
+// src [rows][k] bytes -> dst [rows][ld] (ld a multiple of 16), zero in [k, ld):
+// one thread per 16 bytes, whole chunks as one load at any alignment.
+__global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t *__restrict__ src, int64_t k, int32_t chunks,
+                                                       int64_t total, int8_t *__restrict__ dst) {
   for (int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; q < total;
        q += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t col = q % ld, rr = q / ld;  // rr = c * rows + row
-    dst[q] = col < k ? src[rr * k + col] : static_cast<int8_t>(0);
+    const int64_t row = q / chunks;
+    const int64_t k0 = (q - row * chunks) * 16;
+    const int8_t *from = src + row * k + k0;
+    i32x4 w = {0, 0, 0, 0};
+    if (k0 + 16 <= k) {
+      __builtin_memcpy(&w, from, 16);
+    } else {
+      static_for<16>([&](auto B) {
+        constexpr int b = decltype(B)::value;
+        if (k0 + b < k) w[b / 4] |= static_cast<int32_t>((static_cast<uint32_t>(from[b]) & 0xFFu) << (8 * (b % 4)));
+      });
+    }
+    *reinterpret_cast<i32x4 *>(dst + q * 16) = w;
   }
 }
 
@@ -1305,6 +1378,14 @@ static int32_t packed_plan_from(const rnsmx_plan_t *plan, const GemmArgs &g, Gem
   return RNSMX_OK;
 }
 
+// rows x k bytes -> rows x ld bytes, zero padded.
+static int32_t launch_pad_rows(const int8_t *src, int64_t rows, int64_t k, int64_t ld, int8_t *dst, hipStream_t st) {
+  const int64_t total = rows * (ld / 16);
+  const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 16384));
+  hipLaunchKernelGGL(pad_rows_kernel, dim3(blocks), dim3(256), 0, st, src, k, static_cast<int32_t>(ld / 16), total, dst);
+  return check_launch("pad_rows");
+}
+
 static size_t dtype_size(int32_t dtype) {
   switch (dtype) {
     case RNSMX_INT8: return 1;
@@ -1532,15 +1613,16 @@ int32_t rnsmx_encode_centered(const void *values_dev, int32_t dtype, int64_t row
 }
 
 // The fields of GemmArgs the kernel choice reads, for an M x N x K product
-// (raw int8 activations read in place with row stride K, or residue planes
-// padded to kp).
+// (raw int8 activations read in place with row stride K where that is a
+// multiple of 16, else copied to rows of kp bytes; or residue planes padded to
+// kp).
 static GemmArgs plan_args(int64_t m, int64_t n, int64_t k, int32_t channels, bool araw) {
   GemmArgs g{};
   g.m = static_cast<int32_t>(m);
   g.n = static_cast<int32_t>(n);
   g.kp = static_cast<int32_t>(round_up(std::max<int64_t>(k, 1), RNSMX_K_ALIGN));
-  g.a_k = araw ? static_cast<int32_t>(k) : g.kp;
-  g.a_ld = araw ? k : g.kp;
+  g.a_k = araw && k % 16 == 0 ? static_cast<int32_t>(k) : g.kp;
+  g.a_ld = g.a_k;
   g.mods.channels = channels;
   return g;
 }
@@ -1607,11 +1689,7 @@ int32_t rnsmx_matmul_centered_fused_out(const int8_t *a_dev, const int8_t *b_dev
     // rows of 16-byte chunks are read straight from the caller's planes
     // otherwise (chunks past K load as zero)
     int8_t *a_pad = ws + l.a_pad;
-    const int64_t total = R * static_cast<int64_t>(m) * kp;
-    const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 16384));
-    hipLaunchKernelGGL(pad_rows_kernel, dim3(blocks), dim3(256), 0, st, a_dev, static_cast<int64_t>(m),
-                       static_cast<int64_t>(k), kp, total, a_pad);
-    if (int32_t rc = check_launch("pad_rows")) return rc;
+    if (int32_t rc = launch_pad_rows(a_dev, R * static_cast<int64_t>(m), k, kp, a_pad, st)) return rc;
     a_use = a_pad;
     a_ld = kp;
     a_k = kp;
@@ -1709,10 +1787,11 @@ struct PreparedLayout {
   int64_t a_res, row_l1, xchg, total;
 };
 
-static PreparedLayout prepared_layout(bool araw, int64_t m, int64_t kp, int32_t channels, int64_t xchg) {
+static PreparedLayout prepared_layout(bool araw, int64_t m, int64_t k, int32_t channels, int64_t xchg) {
   PreparedLayout l{};
+  const int64_t kp = round_up(std::max<int64_t>(k, 1), RNSMX_K_ALIGN);
   l.a_res = kTicketBytes;
-  l.row_l1 = l.a_res + (araw ? 0 : round_up(channels * m * kp, 256));
+  l.row_l1 = l.a_res + (araw && k % 16 == 0 ? 0 : round_up((araw ? 1 : channels) * m * kp, 256));
   l.xchg = l.row_l1 + round_up(8 * (m + 1), 256);  // the norms, then their maximum
   l.total = l.xchg + xchg;
   return l;
@@ -1739,14 +1818,24 @@ static PreparedLayout packed_layout(int64_t m, int64_t kp, int32_t channels, int
 // place (araw) or as residue planes.
 static int64_t prepared_need(bool araw, int64_t m, int64_t k, int64_t n, int32_t channels,
                              const rnsmx_plan_t *plan) {
-  const int64_t kp = round_up(std::max<int64_t>(k, 1), RNSMX_K_ALIGN);
   int64_t xchg = 0;
   if (m > 0 && n > 0) {
     const GemmArgs g = plan_args(m, n, k, channels, araw);
     GemmChoice c{};
     if (plan_from(plan, g, araw, true, c) == RNSMX_OK) xchg = xchg_bytes(c, g);
   }
-  return prepared_layout(araw, m, kp, channels, xchg).total;
+  return prepared_layout(araw, m, k, channels, xchg).total;
+}
+
+// Whether int8 activations enter the MFMA as they are (each is its own
+// representative mod every m_c) rather than as residue planes: where the raw
+// sums fit int32.  Rows of K bytes that are not 16-byte aligned are copied to
+// padded ones first, one plane instead of R (4 channels: 146 x 797 x 9536 23.6
+// -> 14.9 us, 141 x 2445 x 12160 78 -> 51); a forced plan names a kernel for one of the two forms and
+// keeps the planes there.
+static bool raw_route(int32_t a_dtype, int64_t k, const rnsmx_moduli_t &mods, const rnsmx_plan_t *plan) {
+  const bool automatic = plan == nullptr || plan->kind == kAuto;
+  return a_dtype == RNSMX_INT8 && raw_accumulator_fits(mods, k) && (k % 16 == 0 || automatic);
 }
 
 int64_t rnsmx_prepared_workspace_bytes(int64_t m, int64_t k, int64_t n, int32_t channels,
@@ -1793,17 +1882,18 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   const int R = mods->channels;
   const int64_t kp = round_up(k, RNSMX_K_ALIGN);
 
-  // int8 activations with 16-byte rows feed the MFMA directly (they are
-  // their own representatives mod every m_c); the encoder then only runs for
-  // the adaptive row L1 norms.  Other sources are encoded to residue planes.
-  const bool araw = !packed && a_dtype == RNSMX_INT8 && k % 16 == 0 && raw_accumulator_fits(*mods, k);
+  // int8 activations feed the MFMA directly (raw_route); the encoder then
+  // only runs for the adaptive row L1 norms.  Other sources are encoded to
+  // residue planes.
+  const bool araw = !packed && raw_route(a_dtype, k, *mods, plan);
+  const bool pad_a = araw && k % 16 != 0;
   GemmArgs g = plan_args(m, n, k, R, araw);
   g.mods = *mods;
   GemmChoice c{};
   if (int32_t rc = packed ? packed_plan_from(plan, g, c, a_dtype) : plan_from(plan, g, araw, true, c)) return rc;
   const bool bytes = c.kind == kBytesRows || c.kind == kBytesLds;
   const PreparedLayout l = packed ? packed_layout(m, kp, R, xchg_bytes(c, g))
-                                  : prepared_layout(araw, m, kp, R, xchg_bytes(c, g));
+                                  : prepared_layout(araw, m, k, R, xchg_bytes(c, g));
   if (workspace_bytes < l.total) {
     set_error("workspace too small: %lld < %lld bytes", static_cast<long long>(workspace_bytes),
               static_cast<long long>(l.total));
@@ -1819,10 +1909,15 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   const bool l1_fold = araw && min_ch != 0 && !l1_in_gemm && m > kAdaptiveFoldInGemm;
   // row_l1_max_kernel's workgroups: their maxima are the words the GEMM folds
   const int l1_groups = static_cast<int>(std::min<int64_t>((m + 3) / 4, kAdaptiveFoldInGemm));
+  const int8_t *a_raw = static_cast<const int8_t *>(a_dev);
+  if (pad_a) {
+    if (int32_t rc = launch_pad_rows(a_raw, m, k, kp, a_res, st)) return rc;
+    a_raw = a_res;
+  }
   EncodeArgs e{};
-  e.values = a_dev;
+  e.values = pad_a ? a_res : a_dev;
   e.rows = m;
-  e.cols = k;
+  e.cols = pad_a ? kp : k;
   e.out_ld = kp;
   e.plane = static_cast<int64_t>(m) * kp;
   e.out = araw ? nullptr : a_res;
@@ -1837,10 +1932,7 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
     g.a = static_cast<const int8_t *>(a_dev);
     g.a_ld = g.a_k = k;
     if (static_cast<int64_t>(k) * ab % 16 != 0) {
-      const int64_t total = static_cast<int64_t>(m) * kp * ab;
-      hipLaunchKernelGGL(pad_rows_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, g.a,
-                         static_cast<int64_t>(m), static_cast<int64_t>(k) * ab, kp * ab, total, a_res);
-      if (int32_t rc = check_launch("pad_rows")) return rc;
+      if (int32_t rc = launch_pad_rows(g.a, m, static_cast<int64_t>(k) * ab, kp * ab, a_res, st)) return rc;
       g.a = a_res;
       g.a_ld = kp;
       g.a_k = static_cast<int32_t>(kp);
@@ -1898,7 +1990,7 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   if (bytes) {
     // set above
   } else if (araw) {
-    g.a = static_cast<const int8_t *>(a_dev);
+    g.a = a_raw;
     g.a_cs = 0;
   } else {
     g.a = a_res;
@@ -1920,6 +2012,69 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   g.w_scale = epilogue ? epilogue->w_scale_dev : nullptr;
   g.bias = epilogue ? epilogue->bias_dev : nullptr;
   return launch_gemm(g, bytes ? ab == 1 : araw, c, reinterpret_cast<uint32_t *>(ws), ws + l.xchg, st, packed);
+}
+
+// Workspace of rnsmx_matmul_wide: that of the prepared-weight product, then the
+// encoded weight.
+static int64_t wide_weight_at(int64_t m, int64_t k, int64_t n, int32_t channels) {
+  const int64_t need = rnsmx_prepared_workspace_bytes(m, k, n, channels, nullptr);
+  return need < 0 ? -1 : round_up(need, 256);
+}
+
+int64_t rnsmx_wide_workspace_bytes(int64_t m, int64_t k, int64_t n, int32_t channels) {
+  const int64_t at = wide_weight_at(m, k, n, channels);
+  if (at < 0) return -1;
+  return at + channels * ((n + 15) / 16) * 16 * round_up(std::max<int64_t>(k, 1), RNSMX_K_ALIGN);
+}
+
+int32_t rnsmx_matmul_wide(const void *a_dev, const void *b_dev, int32_t dtype, int32_t m, int32_t k, int32_t n,
+                          const rnsmx_moduli_t *mods, void *workspace_dev, int64_t workspace_bytes, int64_t *out_dev,
+                          void *stream) {
+  clear_error();
+  if (!mods || mods->channels < 1) return fail(RNSMX_EINVAL, "moduli are not initialised");
+  if (m < 0 || k < 1 || n < 0) return fail(RNSMX_EINVAL, "bad GEMM shape");
+  if (dtype_size(dtype) == 0) return fail(RNSMX_EINVAL, "operands must be int8, int16 or int32");
+  if (!accumulator_fits(*mods, k))
+    return fail(RNSMX_ERANGE, "K * max(floor(m/2))^2 exceeds the int32 accumulator");
+  if (m == 0 || n == 0) return RNSMX_OK;
+  if (!a_dev || !b_dev || !out_dev || !workspace_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
+  if (!aligned16(a_dev)) return fail(RNSMX_EINVAL, "activations must be 16-byte aligned");
+  const int64_t need = rnsmx_wide_workspace_bytes(m, k, n, mods->channels);
+  if (need < 0) return fail(RNSMX_EINVAL, "bad GEMM shape");
+  if (workspace_bytes < need) {
+    set_error("workspace too small: %lld < %lld bytes", static_cast<long long>(workspace_bytes),
+              static_cast<long long>(need));
+    return RNSMX_ESPACE;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t at = wide_weight_at(m, k, n, mods->channels);
+  int8_t *ws = static_cast<int8_t *>(workspace_dev);
+  // the counters of the split that the product will take are cleared by the
+  // encoder, so the workspace may hold anything before the call
+  const bool araw = raw_route(dtype, k, *mods, nullptr);
+  const GemmArgs g = plan_args(m, n, k, mods->channels, araw);
+  const GemmChoice c = auto_plan(g, araw, true);
+  const GemmGrid gr = gemm_grid(c, m, n);
+  const int64_t ntickets = c.splits > 1 ? (gr.tiles - whole_tiles(c, gr.tiles)) * gr.waves : 0;
+  const int64_t kp = round_up(k, RNSMX_K_ALIGN), n16 = (static_cast<int64_t>(n) + 15) / 16;
+  EncodeArgs e{};
+  e.values = b_dev;
+  e.rows = n;
+  e.cols = k;
+  e.out_ld = kp;
+  e.plane = n16 * kp * 16;
+  e.out = ws + at;
+  e.mods = *mods;
+  const dim3 grid(static_cast<unsigned>((n16 + 3) / 4), static_cast<unsigned>(kp / 64)), block(256);
+  uint32_t *tickets = reinterpret_cast<uint32_t *>(ws);
+  switch (dtype) {
+    case RNSMX_INT8: hipLaunchKernelGGL(encode_frag_kn_kernel<int8_t>, grid, block, 0, st, e, tickets, ntickets); break;
+    case RNSMX_INT16: hipLaunchKernelGGL(encode_frag_kn_kernel<int16_t>, grid, block, 0, st, e, tickets, ntickets); break;
+    default: hipLaunchKernelGGL(encode_frag_kn_kernel<int32_t>, grid, block, 0, st, e, tickets, ntickets); break;
+  }
+  if (int32_t rc = check_launch("encode_frag_kn")) return rc;
+  return run_prepared(a_dev, dtype, m, k, n, ws + at, mods, nullptr, 0, nullptr, nullptr, nullptr, ws, at, out_dev,
+                      stream, false);
 }
 
 int64_t rnsmx_packed_workspace_bytes(int64_t m, int64_t k, int64_t n, int32_t channels,
@@ -2002,19 +2157,21 @@ int32_t rnsmx_matmul_prepared_fused_noalloc(const void *a_dev, int32_t a_dtype, 
   // split K over workgroups, whose exchange area can outgrow the static
   // scratch where the same product unsplit fits (an LDS-kernel tail split
   // at K = 4096, N = 12288 needs 16 MiB of exchange); it then runs unsplit.
-  const bool araw = a_dtype == RNSMX_INT8 && k % 16 == 0 && raw_accumulator_fits(*mods, k);
+  const bool araw = raw_route(a_dtype, k, *mods, plan);
   const GemmArgs g = plan_args(m, n, k, mods->channels, araw);
-  const int64_t kp = round_up(k, RNSMX_K_ALIGN);
   GemmChoice c{};
   if (int32_t rc = plan_from(plan, g, araw, true, c)) return rc;
   rnsmx_plan_t own{};
   const rnsmx_plan_t *run_plan = plan;
-  int64_t need = prepared_layout(araw, m, kp, mods->channels, xchg_bytes(c, g)).total;
+  int64_t need = prepared_layout(araw, m, k, mods->channels, xchg_bytes(c, g)).total;
   if (need > RNSMX_NOALLOC_SCRATCH_BYTES && (plan == nullptr || plan->kind == kAuto)) {
-    c = auto_plan(g, araw, false);
+    // as a forced plan, so in the form raw_route gives those
+    own = rnsmx_plan_t{kStream, 1, 1, 1, 1, 0};
+    const bool raw = raw_route(a_dtype, k, *mods, &own);
+    c = auto_plan(plan_args(m, n, k, mods->channels, raw), raw, false);
     own = rnsmx_plan_t{c.kind, c.mb, c.nb, c.ks, 1, 0};
     run_plan = &own;
-    need = prepared_layout(araw, m, kp, mods->channels, 0).total;
+    need = prepared_layout(raw, m, k, mods->channels, 0).total;
   }
   if (need > RNSMX_NOALLOC_SCRATCH_BYTES) {
     set_error("this call needs %lld bytes of scratch; the static scratch holds %lld (use "

@@ -35,6 +35,8 @@ EXPORTED_SYMBOLS = (
     "rnsmx_prepare_weight",
     "rnsmx_prepared_workspace_bytes",
     "rnsmx_matmul_prepared_fused",
+    "rnsmx_wide_workspace_bytes",
+    "rnsmx_matmul_wide",
     "rnsmx_matmul_prepared_fused_noalloc",
     "rnsmx_matmul_residues_prepared",
     "rnsmx_gemm_plan",
@@ -139,6 +141,8 @@ _SIGNATURES = {
         _I32, [_P, _I32, _I32, _I32, _I32, _P, ctypes.POINTER(Moduli), _P, _I32,
                ctypes.POINTER(Adaptive), ctypes.POINTER(Epilogue), ctypes.POINTER(Plan),
                _P, _I64, _P, _P]),
+    "rnsmx_wide_workspace_bytes": (_I64, [_I64, _I64, _I64, _I32]),
+    "rnsmx_matmul_wide": (_I32, [_P, _P, _I32, _I32, _I32, _I32, ctypes.POINTER(Moduli), _P, _I64, _P, _P]),
     "rnsmx_matmul_prepared_fused_noalloc": (
         _I32, [_P, _I32, _I32, _I32, _I32, _P, ctypes.POINTER(Moduli), _P, _I32,
                ctypes.POINTER(Adaptive), ctypes.POINTER(Epilogue), ctypes.POINTER(Plan), _P, _P]),

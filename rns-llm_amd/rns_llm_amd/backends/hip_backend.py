@@ -1008,9 +1008,51 @@ class HipRNSBackend:
         mods = validate_moduli(moduli)
         return self.encode_centered(a, mods), self.encode_centered(b, mods), mods
 
+    def _wide_operands(self, a: torch.Tensor, b: torch.Tensor, moduli: Iterable[int]):
+        """The moduli when one library call (``rnsmx_matmul_wide``) serves the
+        integer pair a [M, K], b [K, N]; None when the chain through residue
+        planes has to (empty operands, two devices) or has to refuse it."""
+        if not (a.is_cuda and b.is_cuda and a.ndim == 2 and b.ndim == 2 and a.is_contiguous() and b.is_contiguous()
+                and a.dtype == b.dtype and a.dtype in _DTYPE_MAX_ABS and a.device == b.device
+                and a.shape[1] == b.shape[0] and a.numel() and b.numel()):
+            return None
+        mods = tuple(moduli)
+        if not self.mfma_compatible(k=int(a.shape[1]), n=int(b.shape[1]), moduli=mods, device=a.device):
+            return None
+        return mods
+
+    def _wide_call(self, a: torch.Tensor, b: torch.Tensor, mods: tuple[int, ...], scratch: torch.Tensor,
+                   out: torch.Tensor) -> torch.Tensor:
+        consts = self._constants(a.device, mods)
+        (m, k), n = a.shape, b.shape[1]
+        self._stats["encode_centered_calls"] += 2
+        self._stats["encode_centered_values"] += int(a.numel()) + int(b.numel())
+        self._stats["fused_gemm_calls"] += 1
+        self._stats[f"fused_gemm_channels_{len(mods)}"] += 1
+        _native.check(self._lib.rnsmx_matmul_wide(
+            _aligned(a).data_ptr(), b.data_ptr(), _native.dtype_code(a.dtype), m, k, n, consts.native_ref,
+            scratch.data_ptr(), scratch.numel(), out.data_ptr(), _stream_handle(a.device)))
+        return out
+
+    def _wide_bytes(self, m: int, k: int, n: int, channels: int) -> int:
+        key = ("wide", m, k, n, channels)
+        nbytes = self._ws_bytes.get(key)
+        if nbytes is None:
+            nbytes = int(self._lib.rnsmx_wide_workspace_bytes(m, k, n, channels))
+            if nbytes < 0:
+                raise ValueError("bad workspace shape")
+            self._ws_bytes[key] = nbytes
+        return nbytes
+
     def matmul_wide(self, a: torch.Tensor, b: torch.Tensor, moduli: Iterable[int], *,
                     decode: bool = True, kernel: str = "auto") -> torch.Tensor:
         """Exact a @ b as int64 (decode) or its centered residues [R, M, N]."""
+        moduli = tuple(moduli)
+        mods = self._wide_operands(a, b, moduli) if decode else None
+        if mods is not None:
+            (m, k), n = map(int, a.shape), int(b.shape[1])
+            scratch = torch.empty((self._wide_bytes(m, k, n, len(mods)),), dtype=torch.uint8, device=a.device)
+            return self._wide_call(a, b, mods, scratch, torch.empty((m, n), dtype=torch.int64, device=a.device))
         a_res, b_res, mods = self._encode_operands(a, b, moduli)
         if not decode:
             return self.matmul_centered_residues(a_res, b_res, mods, kernel=kernel)
@@ -1021,6 +1063,15 @@ class HipRNSBackend:
                           workspace: RNSWorkspace | None = None) -> torch.Tensor:
         """Exact a @ b into ``workspace.output`` (aliasing it, like
         ``matmul_centered_fused``)."""
+        moduli = tuple(moduli)
+        mods = self._wide_operands(a, b, moduli)
+        if mods is not None and lut_channels in (0, 1, 2) and lut_channels <= len(mods):
+            (m, k), n = map(int, a.shape), int(b.shape[1])
+            if workspace is None:
+                workspace = self.create_workspace(device=a.device, channels=len(mods), m=m, n=n)
+            self._check_workspace(workspace, channels=len(mods), m=m, n=n, device=a.device)
+            scratch = self._scratch(workspace, self._wide_bytes(m, k, n, len(mods)))
+            return self._wide_call(a, b, mods, scratch, workspace.output)
         a_res, b_res, mods = self._encode_operands(a, b, moduli)
         return self.matmul_centered_fused(a_res, b_res, mods, lut_channels=lut_channels, workspace=workspace)
 
