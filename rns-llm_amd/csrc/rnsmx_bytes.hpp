@@ -522,10 +522,11 @@ __global__ __launch_bounds__(64 * WM * WN) void bytes_lds_kernel(const GemmArgsK
     asm volatile("" ::: "memory");
     if (lane == 0) __hip_atomic_store(late.tickets + slot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  auto run = [&](auto OUT) __attribute__((always_inline)) {
+  auto run = [&](auto OUT, auto DT) __attribute__((always_inline)) {
     const bool interior = rw0 + 16 * MI <= m_lim && cw0 + 16 * NJ <= n_lim;
     const bool pairs = decltype(OUT)::value == kOutInt64 && interior && (e.out_ld & 1) == 0 &&
                        (reinterpret_cast<uintptr_t>(e.out) & 15) == 0;
+    const bool quads = interior && float_quads_fit<RCAP>(e);
     static_for<MI>([&](auto I) {
       constexpr int i = decltype(I)::value;
       double rt[4];
@@ -550,6 +551,12 @@ __global__ __launch_bounds__(64 * WM * WN) void bytes_lds_kernel(const GemmArgsK
           int64_t y[4];
           static_for<4>([&](auto TT) { y[TT] = frac_int<RCAP>(centered_mod(e, x[TT]) + kRoundMagic); });
           store_int64_pairs(y, as_global<int64_t>(e.out) + idx + (lane & 14), e.out_ld);
+        } else if (quads) {
+          if constexpr (decltype(OUT)::value == kOutFloat) {
+            float f[4];
+            static_for<4>([&](auto TT) { f[decltype(TT)::value] = static_cast<float>(centered_mod(e, x[TT])); });
+            store_float_quads<RCAP, decltype(DT)::value>(e, f, cscale[j], idx + (lane & 3) * e.out_ld + (lane & 12));
+          }
         } else {
           static_for<4>([&](auto TT) {
             constexpr int t = decltype(TT)::value;
@@ -562,9 +569,11 @@ __global__ __launch_bounds__(64 * WM * WN) void bytes_lds_kernel(const GemmArgsK
     });
   };
   if (e.out_dtype == RNSMX_INT64)
-    run(std::integral_constant<int, kOutInt64>{});
+    run(std::integral_constant<int, kOutInt64>{}, std::integral_constant<int, RNSMX_INT64>{});
   else
-    run(std::integral_constant<int, kOutFloat>{});
+    with_float_type<RCAP>(e, [&](auto DT) __attribute__((always_inline)) {
+      run(std::integral_constant<int, kOutFloat>{}, DT);
+    });
 }
 
 }  // namespace rnsmx

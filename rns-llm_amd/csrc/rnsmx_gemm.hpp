@@ -828,6 +828,14 @@ __device__ __forceinline__ int64_t garner_from_sums(const IntConsts<RCAP> &e, co
   }
 }
 
+// y of one element as a float (from frac_sum's double): the integer rounded
+// as the int64 would be.
+template <int RCAP>
+__device__ __forceinline__ float frac_float(double t) {
+  return RCAP <= 4 ? static_cast<float>(static_cast<int32_t>(__builtin_bit_cast(uint64_t, t)))
+                   : static_cast<float>(t - kRoundMagic);
+}
+
 // The output pointers arrive as generic pointers inside the argument block;
 // naming their address space lets the compiler emit global (not flat)
 // memory instructions.
@@ -916,10 +924,7 @@ __device__ __forceinline__ void finish_element(const Epi<RCAP> &e, int c_act, co
     if constexpr (OUT == kOutInt64) {
       store_value<RCAP, OUT>(e, frac_int<RCAP>(t), idx, cs);
     } else {
-      // the same integer rounded to float the same way
-      const float f = RCAP <= 4 ? static_cast<float>(static_cast<int32_t>(__builtin_bit_cast(uint64_t, t)))
-                                : static_cast<float>(t - kRoundMagic);
-      store_float<RCAP>(e, f, idx, cs);
+      store_float<RCAP>(e, frac_float<RCAP>(t), idx, cs);
     }
   } else {
     store_value<RCAP, OUT>(e, garner_from_sums<RCAP>(e.ic, v, FAST ? RCAP : c_act), idx, cs);
@@ -981,7 +986,85 @@ __device__ __forceinline__ void store_int64_pairs(const int64_t (&y)[4], gptr<in
   __builtin_nontemporal_store(v1, reinterpret_cast<__attribute__((address_space(1))) i64x2 *>(p + 2 * ld));
 }
 
-template <int RCAP, int MI, int NJ>
+// Float outputs of one 16 x 16 block whose four rows per lane are f[0..3] =
+// (float)y (rows 4 (lane >> 4) + t of column lane & 15), written four columns
+// of one row per lane: after the float chain of its own column the quad of
+// lanes transposes its 4 x 4 values (DPP swaps with lane ^ 1, then lane ^ 2),
+// so lane l holds row l & 3 of columns 4 ((lane & 15) >> 2) .. +3, one 8-byte
+// (16-byte) store in place of four of 2 (4) bytes: as for int64 outputs the
+// store instructions a CU has in flight are the bound, not the bytes.  `at`
+// points to that row and column; rows are 8 (16) byte aligned.
+template <int RCAP, int DT>
+__device__ __forceinline__ void store_float_quads(const Epi<RCAP> &e, const float (&f)[4], ColScale cs, int64_t at) {
+  const bool odd = (threadIdx.x & 1) != 0, high = (threadIdx.x & 2) != 0;
+  float x[4];
+  {
+#pragma clang fp contract(off)
+    static_for<4>([&](auto T) {
+      constexpr int t = decltype(T)::value;
+      float v = f[t] * e.a_scale;
+      v = v * cs.w;
+      x[t] = e.bias_ptr != nullptr ? v + cs.b : v;
+    });
+  }
+  static constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E;  // quad_perm [1, 0, 3, 2] and [2, 3, 0, 1]
+  auto swap1 = [](uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kSwap1, 0xF, 0xF, false));
+  };
+  auto swap2 = [](uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kSwap2, 0xF, 0xF, false));
+  };
+  if constexpr (DT == RNSMX_FLOAT32) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    uint32_t w[4];
+    static_for<4>([&](auto T) { w[decltype(T)::value] = __float_as_uint(x[decltype(T)::value]); });
+    const uint32_t ra = swap1(odd ? w[0] : w[1]), rb = swap1(odd ? w[2] : w[3]);
+    // two columns of rows 0 and 2 (even lanes) or 1 and 3
+    const uint32_t a0 = odd ? ra : w[0], a1 = odd ? w[1] : ra, b0 = odd ? rb : w[2], b1 = odd ? w[3] : rb;
+    const uint32_t y0 = swap2(high ? a0 : b0), y1 = swap2(high ? a1 : b1);
+    u32x4 v;
+    v.x = high ? y0 : a0;
+    v.y = high ? y1 : a1;
+    v.z = high ? b0 : y0;
+    v.w = high ? b1 : y1;
+    *reinterpret_cast<gptr<u32x4>>(as_global<float>(e.out) + at) = v;
+  } else {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    uint32_t h[4];
+    static_for<4>([&](auto T) {
+      constexpr int t = decltype(T)::value;
+      h[t] = DT == RNSMX_FLOAT16 ? __half_as_ushort(__float2half_rn(x[t])) : f32_to_bf16_rne(x[t]);
+    });
+    const uint32_t p01 = h[0] | (h[1] << 16), p23 = h[2] | (h[3] << 16);
+    // two columns of row 0 / 2 (even lanes: own low half, neighbour's) or 1 / 3
+    const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
+    const uint32_t a = __builtin_amdgcn_perm(swap1(p01), p01, sel), b = __builtin_amdgcn_perm(swap1(p23), p23, sel);
+    const uint32_t y = swap2(high ? a : b);
+    u32x2 v;
+    v.x = high ? y : a;
+    v.y = high ? b : y;
+    *reinterpret_cast<gptr<u32x2>>(as_global<uint16_t>(e.out) + at) = v;
+  }
+}
+
+// Whether a tile at column c0 (a multiple of 16) can be stored so.
+template <int RCAP>
+__device__ __forceinline__ bool float_quads_fit(const Epi<RCAP> &e) {
+  return e.out_dtype != RNSMX_INT64 && (e.out_ld & 3) == 0 && (reinterpret_cast<uintptr_t>(e.out) & 15) == 0;
+}
+// Calls f(DT) for the float output type.
+template <int RCAP, typename F>
+__device__ __forceinline__ void with_float_type(const Epi<RCAP> &e, F &&f) {
+  if (e.out_dtype == RNSMX_FLOAT16)
+    f(std::integral_constant<int, RNSMX_FLOAT16>{});
+  else if (e.out_dtype == RNSMX_BFLOAT16)
+    f(std::integral_constant<int, RNSMX_BFLOAT16>{});
+  else
+    f(std::integral_constant<int, RNSMX_FLOAT32>{});
+}
+
+// QUADS: float outputs four columns per store where they fit.
+template <int RCAP, int MI, int NJ, bool QUADS = true>
 __device__ __forceinline__ void register_epilogue(KArgs<RCAP> &g, const Epi<RCAP> &e, int c_act,
                                                   const i32x4 (&acc)[RCAP][MI][NJ], int r0, int c0,
                                                   int m_lim, int n_lim, const ColScale (&cs)[NJ]) {
@@ -1014,6 +1097,30 @@ __device__ __forceinline__ void register_epilogue(KArgs<RCAP> &g, const Epi<RCAP
       });
     });
     return;
+  }
+  if constexpr (kFrac<RCAP> && QUADS) {
+    if (interior && float_quads_fit<RCAP>(e)) {
+      const int64_t at0 = static_cast<int64_t>(r0 + 4 * (lane >> 4) + (lane & 3)) * e.out_ld + c0 + (lane & 12);
+      with_float_type<RCAP>(e, [&](auto DT) __attribute__((always_inline)) {
+        static_for<MI>([&](auto I) {
+          constexpr int i = decltype(I)::value;
+          int64_t roff = i * 16 * e.out_ld;
+          pin_sgpr(roff);
+          static_for<NJ>([&](auto J) {
+            constexpr int j = decltype(J)::value;
+            float f[4];
+            static_for<4>([&](auto T) {
+              constexpr int t = decltype(T)::value;
+              int32_t v[RCAP];
+              static_for<RCAP>([&](auto C) { v[decltype(C)::value] = acc[decltype(C)::value][i][j][t]; });
+              f[t] = frac_float<RCAP>(frac_sum<RCAP>(e, v));
+            });
+            store_float_quads<RCAP, decltype(DT)::value>(e, f, cs[j], at0 + roff + j * 16);
+          });
+        });
+      });
+      return;
+    }
   }
   // always inlined: a call would pass the accumulators by reference, i.e.
   // through memory for the whole kernel (the inliner gives up on the
@@ -2730,7 +2837,10 @@ __device__ __forceinline__ void lds_planes_body(KArgs<RCAP> &g, int8_t *smem, co
     return;
   ColScale cs[NJ];
   static_for<NJ>([&](auto J) { cs[J] = col_scale<RCAP>(e, cw0 + decltype(J)::value * 16 + (lane & 15), n_lim); });
-  register_epilogue<RCAP, MI, NJ>(g, e, c_act, acc, rw0, cw0, m_lim, n_lim, cs);
+  // without the quad stores at 6 channels: with them the register allocator
+  // spills four accumulators inside the loop (512 x 4096 x 12288: 210 us
+  // against 190)
+  register_epilogue<RCAP, MI, NJ, RCAP == 4>(g, e, c_act, acc, rw0, cw0, m_lim, n_lim, cs);
 }
 
 // Work unit of workgroup blockIdx.x for the residue-plane kernel.  Tile t

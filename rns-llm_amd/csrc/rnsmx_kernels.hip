@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256) void encode_frag_kernel(const EncodeArgs e) {
 template <typename T>
 __global__ __launch_bounds__(256) void encode_frag_kn_kernel(const EncodeArgs e, uint32_t *tickets, int64_t ntickets) {
   constexpr int kRow = 64 + 4 / sizeof(T);  // one bank of padding
-  __shared__ T tile[64 * kRow];
+  __shared__ __attribute__((aligned(16))) T tile[64 * kRow];
   for (int64_t q = (static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x; q < ntickets;
        q += static_cast<int64_t>(gridDim.x) * gridDim.y * 256)
     tickets[q] = 0;
@@ -295,16 +295,20 @@ __global__ __launch_bounds__(256) void encode_frag_kn_kernel(const EncodeArgs e,
     const int q = decltype(U)::value * 256 + threadIdx.x;
     const int r = q / (64 / V), c = q % (64 / V) * V;
     const int64_t k = ks * 64 + r, col = n0 + c;
-    T v[V];
+    uint32_t w[4];
     if (k < e.cols && col + V <= n) {
-      __builtin_memcpy(v, src + k * n + col, 16);
+      __builtin_memcpy(w, src + k * n + col, 16);
     } else {
+      T v[V];
       static_for<V>([&](auto I) {
         constexpr int i = decltype(I)::value;
         v[i] = k < e.cols && col + i < n ? src[k * n + col + i] : static_cast<T>(0);
       });
+      __builtin_memcpy(w, v, 16);
     }
-    __builtin_memcpy(&tile[r * kRow + c], v, 16);
+    // rows are whole dwords but not whole 16-byte chunks
+    uint32_t *to = reinterpret_cast<uint32_t *>(&tile[r * kRow + c]);
+    static_for<4>([&](auto D) { to[decltype(D)::value] = w[decltype(D)::value]; });
   });
   __syncthreads();
   const int64_t jb = static_cast<int64_t>(blockIdx.x) * 4 + wave;

@@ -135,3 +135,31 @@ def test_shorter_prefixes(backend, m, moduli, dtype, expect):
     out, meta = backend.matmul_prepared_adaptive_fused(a.cuda(), adaptive, return_metadata=True)
     assert meta["channels"] == expect and meta["bound"] == bound
     assert torch.equal(out.cpu(), torch.from_numpy(ro.exact_matmul(a.numpy(), w.t().numpy())))
+
+
+# float outputs: whole tiles with rows of 4 columns (four columns per store),
+# rows of 66 and 70 (one column per store) and edges, every tile family
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [64, 66, 70, 100, 192])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("plan,dtype", [((2, 2, 1, 0), torch.int8), ((5, 3, 1, 4), torch.int8), ((3, 0, 0, 0), torch.int8),
+                                        ((7, 0, 0, 0), torch.int8), ((8, 0, 0, 0), torch.int16)], ids=str)
+def test_float_rows(backend, plan, dtype, out_dtype, n):
+    m, k = 261, 256
+    moduli = (255, 253, 251, 247) if dtype == torch.int8 else (255, 253, 251, 247, 241, 239)
+    gen = torch.Generator().manual_seed(n)
+    lim = 128 if dtype == torch.int8 else 32768
+    a = torch.randint(-lim, lim, (m, k), generator=gen, dtype=torch.int32).to(dtype)
+    w = torch.randint(-lim, lim, (n, k), generator=gen, dtype=torch.int32).to(dtype)
+    scale, w_scale = torch.tensor([1e-3]), torch.rand((n,), generator=gen) * 1e-3
+    bias = torch.randn((n,), generator=gen)
+    prepared = backend.prepare_weight_nk(w.cuda(), moduli)
+    exact = torch.from_numpy(ro.exact_matmul(a.numpy(), w.t().numpy()))
+    for b in (bias, None):
+        out = torch.empty((m, n), dtype=out_dtype, device="cuda")
+        backend.matmul_prepared_fused(a.cuda(), prepared, plan=plan, out=out, a_scale=scale.cuda(), w_scale=w_scale.cuda(),
+                                      bias=None if b is None else b.cuda())
+        ref = (exact.float() * scale.view(1, 1)) * w_scale.unsqueeze(0)
+        ref = (ref if b is None else ref + b).to(out_dtype)
+        bits = torch.int32 if out_dtype == torch.float32 else torch.int16
+        assert torch.equal(out.cpu().view(bits), ref.view(bits))
