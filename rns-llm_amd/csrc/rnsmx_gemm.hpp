@@ -74,10 +74,12 @@ struct GemmMods {
   int32_t channels;
   uint32_t moduli[RCAP];
   uint32_t magic[RCAP];
-  uint32_t qinv[RCAP];
-  int32_t qk16[RCAP];
-  uint32_t qk8[RCAP];
-  uint32_t ucoef[RCAP][RCAP];
+  // the mixed-radix digits' constants (past 6 channels only)
+  static constexpr int kDigits = kFrac<RCAP> ? 1 : RCAP;
+  uint32_t qinv[kDigits];
+  int32_t qk16[kDigits];
+  uint32_t qk8[kDigits];
+  uint32_t ucoef[kDigits][kDigits];
   int64_t prefix[RCAP + 1];
   double frac[kFrac<RCAP> ? kFracParts<RCAP> : 1][kFrac<RCAP> ? RCAP : 1];
   double p_full, turn, magic_p;
@@ -136,10 +138,12 @@ inline GemmArgsK<RCAP> compact_args(const GemmArgs &g) {
   for (int c = 0; c < RCAP && c < RNSMX_MAX_CHANNELS; ++c) {
     k.mods.moduli[c] = static_cast<uint32_t>(f.moduli[c]);
     k.mods.magic[c] = f.magic[c];
-    k.mods.qinv[c] = f.qinv[c];
-    k.mods.qk16[c] = f.qk16[c];
-    k.mods.qk8[c] = f.qk8[c];
-    for (int j = 0; j < RCAP && j < RNSMX_MAX_CHANNELS; ++j) k.mods.ucoef[j][c] = f.ucoef[j][c];
+    if constexpr (!kFrac<RCAP>) {
+      k.mods.qinv[c] = f.qinv[c];
+      k.mods.qk16[c] = f.qk16[c];
+      k.mods.qk8[c] = f.qk8[c];
+      for (int j = 0; j < RCAP && j < RNSMX_MAX_CHANNELS; ++j) k.mods.ucoef[j][c] = f.ucoef[j][c];
+    }
   }
   for (int c = 0; c <= RCAP && c <= RNSMX_MAX_CHANNELS; ++c) k.mods.prefix[c] = f.prefix[c];
   if constexpr (kFrac<RCAP>) {
@@ -476,7 +480,7 @@ struct IntConsts {
 // scalar loads at their first use in the epilogue, where each dependent
 // round of scalar-cache misses is exposed.  The integer constants are read
 // here only past 6 channels; elsewhere by the K split's exchange, the one
-// path that needs them (int_consts).
+// path that needs them (residue_consts).
 template <int RCAP>
 struct Epi {
   double f[kFrac<RCAP> ? kFracParts<RCAP> : 1][RCAP];  // rows of frac_sum for the active prefix
@@ -490,23 +494,31 @@ struct Epi {
   float a_scale;
 };
 
-// IntConsts from a moduli block (kernel arguments or a by-value copy).
+// IntConsts from a moduli block (kernel arguments or a by-value copy): those
+// of the residues (reduce_acc), then those of the digits too.
 template <int RCAP, typename Mods>
-__device__ __forceinline__ void fill_moduli(IntConsts<RCAP> &e, const Mods &mods, int c_act) {
+__device__ __forceinline__ void fill_residues(IntConsts<RCAP> &e, const Mods &mods) {
   static_for<RCAP>([&](auto C) {
     constexpr int c = decltype(C)::value;
     const uint32_t m = static_cast<uint32_t>(mods.moduli[c]), magic = mods.magic[c];
     e.m[c] = m;
-    e.qinv[c] = mods.qinv[c];
-    e.qk16[c] = mods.qk16[c];
-    e.qk8[c] = mods.qk8[c];
-    static_for<c>([&](auto J) { e.u[decltype(J)::value][c] = mods.ucoef[decltype(J)::value][c]; });
     // the 24-bit reduction constants (see canon_fast); channels past the
     // set's size have m = 0 and are never used
     e.m24[c] = magic >> 8;
     e.c16[c] = 65536u - (magic >> 16) * m;
     e.bias[c] = m * (magic >> 9);
     e.negm[c] = -static_cast<int32_t>(m);
+  });
+}
+template <int RCAP, typename Mods>
+__device__ __forceinline__ void fill_moduli(IntConsts<RCAP> &e, const Mods &mods, int c_act) {
+  fill_residues<RCAP>(e, mods);
+  static_for<RCAP>([&](auto C) {
+    constexpr int c = decltype(C)::value;
+    e.qinv[c] = mods.qinv[c];
+    e.qk16[c] = mods.qk16[c];
+    e.qk8[c] = mods.qk8[c];
+    static_for<c>([&](auto J) { e.u[decltype(J)::value][c] = mods.ucoef[decltype(J)::value][c]; });
   });
   static_for<RCAP + 1>([&](auto C) { e.prefix[decltype(C)::value] = mods.prefix[decltype(C)::value]; });
   e.p_act = prefix_at<RCAP>(mods, c_act);
@@ -701,13 +713,13 @@ __device__ __forceinline__ void pin_epi(Epi<RCAP> &e) {
   pin_sgpr(e.bias_ptr);
 }
 
-// The integer constants for a path that needs them: read here where
-// load_epi did not.
+// The residue constants for the K split's exchange: read here where load_epi
+// did not.
 template <int RCAP>
-__device__ __forceinline__ IntConsts<RCAP> int_consts(KArgs<RCAP> &g, const Epi<RCAP> &e, int c_act) {
+__device__ __forceinline__ IntConsts<RCAP> residue_consts(KArgs<RCAP> &g, const Epi<RCAP> &e) {
   if constexpr (kFrac<RCAP>) {
     IntConsts<RCAP> ic;
-    fill_moduli<RCAP>(ic, g.mods, c_act);
+    fill_residues<RCAP>(ic, g.mods);
     return ic;
   } else {
     return e.ic;
@@ -1354,7 +1366,7 @@ __device__ __forceinline__ bool split_exchange(KArgs<RCAP> &g, const Epi<RCAP> &
   constexpr int CH = MI * NJ * XW;  // 1 KB blocks per wave and split
   const int lane = threadIdx.x & 63;
   const int S = g.splits;
-  const IntConsts<RCAP> ic = int_consts<RCAP>(g, e, 0);
+  const IntConsts<RCAP> ic = residue_consts<RCAP>(g, e);
   int8_t *base = g.xchg + slot * S * CH * 1024 + lane * 4;
   auto block = [&](int s, int i, int j, int wd) {
     return base + (static_cast<int64_t>(s) * CH + (i * NJ + j) * XW + wd) * 1024;

@@ -20,6 +20,7 @@
 
 #include "rnsmx_bytes.hpp"
 #include "rnsmx_gemm.hpp"
+#include "rnsmx_quant.hpp"
 
 namespace rnsmx {
 
@@ -1425,68 +1426,6 @@ static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 // 3 us: below this size the saved launch is worth more.
 static constexpr int64_t kQuantOneBlockMax = 16384;
 
-struct QuantArgs {
-  const void *x;
-  int64_t count;
-  int32_t vec;      // 1: x is 16-byte aligned, read in 16-byte vectors
-  int32_t nparts;   // blocks of the amax pass
-  float qmax, rcp;  // rcp = fl32(1 / qmax)
-  float *partial;
-  float *scale;
-  void *q;
-};
-
-// Input element decoding: float32, or the bits of a float16 / bfloat16.
-template <typename T>
-struct QuantIn;
-template <>
-struct QuantIn<float> {
-  __device__ static float get(float v) { return v; }
-};
-struct Bf16Bits {
-  uint16_t bits;
-};
-template <>
-struct QuantIn<__half> {
-  __device__ static float get(uint16_t v) { return __half2float(__ushort_as_half(v)); }
-};
-template <>
-struct QuantIn<Bf16Bits> {
-  __device__ static float get(uint16_t v) { return __uint_as_float(static_cast<uint32_t>(v) << 16); }
-};
-template <typename T>
-using QuantRaw = typename std::conditional<std::is_same<T, float>::value, float, uint16_t>::type;
-
-
-
-// max(a, b) that propagates NaN, as torch's amax does (fmaxf drops it).
-__device__ __forceinline__ float max_nan(float a, float b) {
-  return (a != a || b != b) ? __builtin_nanf("") : fmaxf(a, b);
-}
-
-// max |x| over the elements this thread visits (tid, tid + stride, ...);
-// NaN when any of them is NaN.
-template <typename T>
-__device__ __forceinline__ float quant_thread_amax(const QuantArgs &a, int64_t tid, int64_t stride) {
-  using R = QuantRaw<T>;
-  constexpr int V = 16 / sizeof(R);
-  const R *x = static_cast<const R *>(a.x);
-  const int64_t nvec = a.vec ? a.count / V : 0;
-  float m = 0.0f;
-  bool nan = false;
-  auto visit = [&](float v) {
-    m = fmaxf(m, fabsf(v));
-    nan |= v != v;
-  };
-  for (int64_t i = tid; i < nvec; i += stride) {
-    R v[V];
-    *reinterpret_cast<uint4 *>(v) = reinterpret_cast<const uint4 *>(x)[i];
-    static_for<V>([&](auto E) { visit(QuantIn<T>::get(v[decltype(E)::value])); });
-  }
-  for (int64_t i = nvec * V + tid; i < a.count; i += stride) visit(QuantIn<T>::get(x[i]));
-  return nan ? __builtin_nanf("") : m;
-}
-
 // q = clamp(rint(x / s), -qmax, qmax) over the elements of (tid, stride).
 template <typename T, typename Q>
 __device__ __forceinline__ void quant_thread_apply(const QuantArgs &a, float s, int64_t tid, int64_t stride) {
@@ -1494,12 +1433,7 @@ __device__ __forceinline__ void quant_thread_apply(const QuantArgs &a, float s, 
   constexpr int V = 16 / sizeof(R);
   const R *x = static_cast<const R *>(a.x);
   Q *q = static_cast<Q *>(a.q);
-  // a NaN quotient (x NaN, s NaN, or x and s infinite) quantizes to 0, the
-  // value the hardware's float-to-integer conversion gives NaN
-  auto quant = [&](R raw) {
-    const float r = rintf(QuantIn<T>::get(raw) / s);
-    return static_cast<Q>(r != r ? 0.0f : fminf(fmaxf(r, -a.qmax), a.qmax));
-  };
+  auto quant = [&](R raw) { return static_cast<Q>(quant_value(QuantIn<T>::get(raw), s, a.qmax)); };
   const int64_t nvec = a.vec ? a.count / V : 0;
   for (int64_t i = tid; i < nvec; i += stride) {
     R v[V];
@@ -1540,8 +1474,7 @@ __global__ __launch_bounds__(256) void quant_apply_kernel(const QuantArgs a) {
   float t = 0.0f;
   for (int b = threadIdx.x; b < a.nparts; b += blockDim.x) t = max_nan(t, a.partial[b]);
   const float amax = block_max256(t, wmax);
-  // clamp at FLT_EPSILON; NaN stays NaN (torch.clamp keeps it, fmaxf would not)
-  const float s = amax != amax ? amax : fmaxf(amax * a.rcp, 1.1920928955078125e-07f);
+  const float s = quant_scale(amax, a.rcp);
   if (blockIdx.x == 0 && threadIdx.x == 0) *a.scale = s;
   quant_thread_apply<T, Q>(a, s, static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x,
                            static_cast<int64_t>(gridDim.x) * blockDim.x);
@@ -1559,8 +1492,7 @@ __global__ __launch_bounds__(1024) void quant_one_block_kernel(const QuantArgs a
   __syncthreads();
   float amax = 0.0f;
   for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) amax = max_nan(amax, wmax[w]);
-  // clamp at FLT_EPSILON; NaN stays NaN (torch.clamp keeps it, fmaxf would not)
-  const float s = amax != amax ? amax : fmaxf(amax * a.rcp, 1.1920928955078125e-07f);
+  const float s = quant_scale(amax, a.rcp);
   if (threadIdx.x == 0) *a.scale = s;
   quant_thread_apply<T, Q>(a, s, threadIdx.x, blockDim.x);
 }
@@ -2374,6 +2306,30 @@ int32_t rnsmx_linear_forward(const void *x_dev, int32_t x_dtype, int32_t rows, i
     set_error("workspace too small: %lld < %lld bytes", static_cast<long long>(workspace_bytes),
               static_cast<long long>(l.total));
     return RNSMX_ESPACE;
+  }
+  if (linear_rows_fits(rows, k, *mods, quant_bits, adaptive != nullptr && adaptive->min_channels != 0) && n > 0) {
+    // a few rows: quantized inside the product, one launch
+    if (!x_dev || !packed_dev || !out_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
+    GemmArgs g = plan_args(rows, n, k, mods->channels, true);
+    g.mods = *mods;
+    g.a_k = k;
+    g.b = packed_dev;
+    g.b_ld = static_cast<int64_t>(g.kp) * 16;
+    g.b_cs = g.b_ld * ((static_cast<int64_t>(n) + 15) / 16);
+    g.out = out_dev;
+    g.out_ld = n;
+    g.out_dtype = x_dtype;
+    g.a_scale = w_scale_dev;  // not read: the scale stays in the kernel
+    g.w_scale = w_scale_dev;
+    g.bias = bias_dev;
+    QuantArgs a{};
+    a.x = x_dev;
+    a.count = static_cast<int64_t>(rows) * k;
+    a.vec = aligned16(x_dev);
+    a.qmax = 127.0f;
+    a.rcp = 1.0f / a.qmax;
+    launch_linear_rows(g, a, x_dtype, static_cast<hipStream_t>(stream));
+    return check_launch("linear_rows");
   }
   int8_t *ws = static_cast<int8_t *>(workspace_dev);
   float *scale = reinterpret_cast<float *>(ws + l.scale);

@@ -1,0 +1,198 @@
+// RNSLinear.forward at decode in one launch: a few rows of float activations
+// are quantized inside the weight-streaming product.
+#include "rnsmx_gemm.hpp"
+#include "rnsmx_quant.hpp"
+
+namespace rnsmx {
+
+// The product's arguments first: kernel_args reads them in place.
+struct LinearRowsArgs {
+  GemmArgsK<4> g;  // m rows of a_k = K values, b, the epilogue
+  QuantArgs q;     // x, vec, qmax, rcp
+};
+
+// A workgroup of 4 waves (3 where K holds no more chunks) owns 16 columns and
+// every row (up to 16), the waves splitting K as in stream_kernel.  The first
+// weight chunk is in flight before anything else; while it travels the
+// workgroup reads all the activations (at most kLinearRowsValues, from L2 after
+// the first), takes their maximum, quantizes them and leaves the int8 rows in
+// LDS (rows of kp + 16 bytes, zero past K, so a fragment's 16 rows do not share
+// banks), from where every K step takes its A fragment.  The next chunk is
+// loaded while one computes.  Quantizing once per workgroup costs less than the
+// launch it saves: the layer at 768 x 2304, 1 row, spent 2.6 of its 13 us on the
+// quantizer's kernel and 3 on its launch.
+// NT: weights with the streaming hint (long K, as stream_kernel).
+constexpr int kLinearRowsMax = 16;
+constexpr int kLinearRowsValues = 8192;
+
+template <typename T, bool NT>
+__global__ __launch_bounds__(256) void linear_rows_kernel(const LinearRowsArgs args) {
+  constexpr int RCAP = 4, U = 4;
+  using R = QuantRaw<T>;
+  constexpr int V = 16 / sizeof(R);
+  constexpr int IT = (kLinearRowsValues / V + 191) / 192;  // vectors per thread (3 waves at least)
+  KArgs<RCAP> &g = kernel_args<GemmArgsK<RCAP>>();
+  const QuantArgs &qa = args.q;
+  prefetch_kernel_args<static_cast<int>(sizeof(LinearRowsArgs))>();
+  __shared__ int32_t sums[RCAP][256];
+  __shared__ float wmax[4];
+  extern __shared__ __attribute__((aligned(16))) int8_t rows_q[];  // [m][kp + 16]
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nthreads = g.threads, ks_n = nthreads >> 6;
+  const int n0 = blockIdx.x * 16, nk = g.kp >> 6, k = g.a_k, m = g.m;
+  const int ldk = g.kp + 16;
+  const int8_t *bp = g.b + static_cast<int64_t>(blockIdx.x) * g.b_ld + lane * 16;
+  const int64_t b_cs = g.b_cs;
+
+  i32x4 fb[2][U][RCAP];
+  auto load_chunk = [&](auto BUF, int q) {
+    static_for<U>([&](auto UU) {
+      const int ks = min(q + decltype(UU)::value, nk - 1);
+      static_for<RCAP>([&](auto C) {
+        const int8_t *p = bp + decltype(C)::value * b_cs + ks * 1024;
+        fb[decltype(BUF)::value][decltype(UU)::value][decltype(C)::value] = NT ? load16_nt(p) : load16(p);
+      });
+    });
+  };
+  constexpr std::integral_constant<int, 0> b0{};
+  constexpr std::integral_constant<int, 1> b1{};
+  int q = wave * U;
+  const int stride = ks_n * U;
+  load_chunk(b0, q);
+
+  // activations: 16-byte vectors kept in registers where rows hold whole ones
+  const R *x = static_cast<const R *>(qa.x);
+  const int count = m * k;
+  const bool vec = qa.vec != 0 && k % V == 0;
+  const int kv = k / V, nvec = m * kv;
+  R v[IT][V];
+  float amax = 0.0f;
+  bool nan = false;
+  auto visit = [&](float f) {
+    amax = fmaxf(amax, fabsf(f));
+    nan |= f != f;
+  };
+  if (vec) {
+    static_for<IT>([&](auto I) {
+      const int i = tid + decltype(I)::value * nthreads;
+      uint4 w = {0u, 0u, 0u, 0u};
+      if (i < nvec) w = reinterpret_cast<const uint4 *>(x)[i];
+      *reinterpret_cast<uint4 *>(v[decltype(I)::value]) = w;
+    });
+  }
+  for (int i = tid; i < RCAP * 256; i += nthreads) (&sums[0][0])[i] = 0;
+  for (int i = tid * 4; i < m * ldk; i += nthreads * 4) *reinterpret_cast<uint32_t *>(rows_q + i) = 0;
+  if (vec) {
+    static_for<IT>([&](auto I) {
+      static_for<V>([&](auto E) { visit(QuantIn<T>::get(v[decltype(I)::value][decltype(E)::value])); });
+    });
+  } else {
+    for (int i = tid; i < count; i += nthreads) visit(QuantIn<T>::get(x[i]));
+  }
+  amax = nan ? __builtin_nanf("") : amax;
+  for (int off = 32; off > 0; off >>= 1) amax = max_nan(amax, __shfl_xor(amax, off, 64));
+  if (lane == 0) wmax[wave] = amax;
+  __syncthreads();
+  amax = wmax[0];
+  for (int w = 1; w < ks_n; ++w) amax = max_nan(amax, wmax[w]);
+  const float s = quant_scale(amax, qa.rcp), qmax = qa.qmax;
+  auto quant = [&](R raw) {
+    return static_cast<uint32_t>(static_cast<int32_t>(quant_value(QuantIn<T>::get(raw), s, qmax))) & 0xFFu;
+  };
+  if (vec) {
+    static_for<IT>([&](auto I) {
+      const int i = tid + decltype(I)::value * nthreads;
+      if (i < nvec) {
+        const int row = i / kv, c = i - row * kv;
+        uint32_t w[V / 4];
+        static_for<V / 4>([&](auto W) {
+          constexpr int e = 4 * decltype(W)::value;
+          const R *r = v[decltype(I)::value];
+          w[decltype(W)::value] = quant(r[e]) | (quant(r[e + 1]) << 8) | (quant(r[e + 2]) << 16) | (quant(r[e + 3]) << 24);
+        });
+        uint32_t *to = reinterpret_cast<uint32_t *>(rows_q + row * ldk + c * V);
+        static_for<V / 4>([&](auto W) { to[decltype(W)::value] = w[decltype(W)::value]; });
+      }
+    });
+  } else {
+    for (int i = tid; i < count; i += nthreads) {
+      const int row = i / k;
+      rows_q[row * ldk + (i - row * k)] = static_cast<int8_t>(quant(x[i]));
+    }
+  }
+  Epi<RCAP> e;
+  load_epi<RCAP>(g, e, g.mods.channels);
+  e.a_scale = s;
+  const int n_lim = g.n;
+  const ColScale cs = col_scale<RCAP>(e, n0 + (tid & 15), n_lim);
+  __syncthreads();
+
+  i32x4 acc[RCAP];
+  static_for<RCAP>([&](auto C) { acc[decltype(C)::value] = acc_zero(); });
+  const int8_t *ap = rows_q + min(lane & 15, m - 1) * ldk + (lane >> 4) * 16;
+  auto mfma_chunk = [&](auto BUF, int at) {
+    static_for<U>([&](auto UU) {
+      constexpr int u = decltype(UU)::value;
+      if (at + u >= nk) return;
+      const i32x4 fa = *reinterpret_cast<const i32x4 *>(ap + (at + u) * 64);
+      static_for<RCAP>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        acc[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, fb[decltype(BUF)::value][u][c], acc[c], 0, 0, 0);
+      });
+    });
+  };
+  while (q < nk) {
+    if (q + stride < nk) load_chunk(b1, q + stride);
+    mfma_chunk(b0, q);
+    q += stride;
+    if (q >= nk) break;
+    if (q + stride < nk) load_chunk(b0, q + stride);
+    mfma_chunk(b1, q);
+    q += stride;
+  }
+  static_for<RCAP>([&](auto C) {
+    static_for<4>([&](auto TT) {
+      constexpr int c = decltype(C)::value, t = decltype(TT)::value;
+      const int r = 4 * (lane >> 4) + t;
+      if (r < m) atomicAdd(&sums[c][r * 16 + (lane & 15)], acc[c][t]);
+    });
+  });
+  __syncthreads();
+  // one element per thread, two trips where three waves serve more than 12 rows
+  for (int at = tid; at < m * 16; at += nthreads) {
+    const int col = n0 + (at & 15);
+    if (col >= n_lim) continue;
+    int32_t sum[RCAP];
+    static_for<RCAP>([&](auto C) { sum[decltype(C)::value] = sums[decltype(C)::value][at]; });
+    store_float<RCAP>(e, frac_float<RCAP>(frac_sum<RCAP>(e, sum)), static_cast<int64_t>(at >> 4) * e.out_ld + col, cs);
+  }
+}
+
+template <typename T>
+static void launch_linear_t(const LinearRowsArgs &a, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>((a.g.n + 15) / 16)), block(static_cast<unsigned>(a.g.threads));
+  const size_t lds = static_cast<size_t>(a.g.m) * (a.g.kp + 16);
+  if (a.g.kp >= 4096)
+    hipLaunchKernelGGL((linear_rows_kernel<T, true>), grid, block, lds, st, a);
+  else
+    hipLaunchKernelGGL((linear_rows_kernel<T, false>), grid, block, lds, st, a);
+}
+
+bool linear_rows_fits(int64_t rows, int64_t k, const rnsmx_moduli_t &mods, int32_t quant_bits, bool adaptive) {
+  return quant_bits == 8 && !adaptive && mods.channels == 4 && rows >= 1 && rows <= kLinearRowsMax &&
+         rows * k <= kLinearRowsValues && raw_accumulator_fits(mods, k);
+}
+
+void launch_linear_rows(const GemmArgs &g, const QuantArgs &q, int32_t x_dtype, hipStream_t st) {
+  LinearRowsArgs a{compact_args<4>(g), q};
+  const int chunks = (g.kp / 64 + 3) / 4;
+  a.g.threads = 64 * (chunks < 4 ? 3 : 4);
+  switch (x_dtype) {
+    case RNSMX_FLOAT16: launch_linear_t<__half>(a, st); break;
+    case RNSMX_BFLOAT16: launch_linear_t<Bf16Bits>(a, st); break;
+    default: launch_linear_t<float>(a, st); break;
+  }
+}
+
+}  // namespace rnsmx
