@@ -237,6 +237,27 @@ int32_t rnsmx_matmul_prepared_fused(
     void *out_dev, void *stream);
 
 /*
+ * Continuous batching: `count` requests, request i holding rows[i] >= 1
+ * contiguous rows of K values (a_dtype) at requests[i] (a host array of device
+ * pointers, any alignment), against one prepared weight (packed_form 0: from
+ * rnsmx_prepare_weight, else rnsmx_prepare_weight_packed): the product of the
+ * rows one after the other -> out_dev [sum rows][N] int64, as
+ * rnsmx_matmul_prepared_fused (rnsmx_matmul_packed_fused) of their
+ * concatenation, which staging_dev ([sum rows][K], 16-byte aligned) holds
+ * afterwards.  Workspace as for that call.  One launch for up to 16 int8 rows
+ * (4 channels, K a multiple of 16, 16-byte aligned requests).
+ * Replaces the concatenation and product of matmul_prepared_fused_requests
+ * (cuda_backend.py:647-703).
+ */
+int32_t rnsmx_matmul_requests(const void *const *requests, const int32_t *rows,
+                              int32_t count, int32_t a_dtype, int32_t k,
+                              int32_t n, const int8_t *packed_dev,
+                              const rnsmx_moduli_t *mods, int32_t packed_form,
+                              void *staging_dev, void *workspace_dev,
+                              int64_t workspace_bytes, int64_t *out_dev,
+                              void *stream);
+
+/*
  * Both operands plain integers, used once: a_dev [M][K] and b_dev [K][N], both
  * int8, int16 or int32 (row-major) -> exact out_dev [M][N] int64.  Encodes B
  * straight into the fragment-major order of rnsmx_prepare_weight in the

@@ -1950,6 +1950,89 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   return launch_gemm(g, bytes ? ab == 1 : araw, c, reinterpret_cast<uint32_t *>(ws), ws + l.xchg, st, packed);
 }
 
+// The requests' rows one after the other: block (x, y) copies 4 KB x of request
+// y (any alignment).
+static constexpr int kGatherMost = 32;  // requests per launch
+struct GatherArgs {
+  const int8_t *from[kGatherMost];
+  int64_t at[kGatherMost + 1];  // byte offsets in `to`
+  int8_t *to;
+};
+__global__ __launch_bounds__(256) void gather_requests_kernel(const GatherArgs args) {
+  RNSMX_KARG(GatherArgs) &a = kernel_args<GatherArgs>();
+  const int r = blockIdx.y;
+  const int64_t at = a.at[r], bytes = a.at[r + 1] - at;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 16;
+  const int8_t *from = a.from[r] + i;
+  int8_t *to = a.to + at + i;
+  if (i + 16 <= bytes) {
+    i32x4 w;
+    __builtin_memcpy(&w, from, 16);
+    __builtin_memcpy(to, &w, 16);
+  } else {
+    for (int64_t b = 0; i + b < bytes; ++b) to[b] = from[b];
+  }
+}
+
+int32_t rnsmx_matmul_requests(const void *const *requests, const int32_t *rows, int32_t count, int32_t a_dtype,
+                              int32_t k, int32_t n, const int8_t *packed_dev, const rnsmx_moduli_t *mods,
+                              int32_t packed_form, void *staging_dev, void *workspace_dev, int64_t workspace_bytes,
+                              int64_t *out_dev, void *stream) {
+  clear_error();
+  if (!mods || mods->channels < 1) return fail(RNSMX_EINVAL, "moduli are not initialised");
+  if (!requests || !rows || count < 1 || k < 1 || n < 0 || dtype_size(a_dtype) == 0)
+    return fail(RNSMX_EINVAL, "bad request batch");
+  if (!staging_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
+  int64_t m = 0;
+  bool aligned = aligned16(staging_dev);
+  for (int32_t i = 0; i < count; ++i) {
+    if (rows[i] < 1 || !requests[i]) return fail(RNSMX_EINVAL, "every request needs a row");
+    m += rows[i];
+    aligned = aligned && aligned16(requests[i]);
+  }
+  if (m > INT32_MAX) return fail(RNSMX_EINVAL, "bad request batch");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  int8_t *staging = static_cast<int8_t *>(staging_dev);
+  if (packed_form == 0 && aligned && n > 0 && request_rows_fits(m, k, *mods, a_dtype)) {
+    if (!packed_dev || !out_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
+    GemmArgs g = plan_args(m, n, k, mods->channels, true);
+    g.mods = *mods;
+    g.b = packed_dev;
+    g.b_ld = static_cast<int64_t>(g.kp) * 16;
+    g.b_cs = g.b_ld * ((static_cast<int64_t>(n) + 15) / 16);
+    g.out = out_dev;
+    g.out_ld = n;
+    g.out_dtype = RNSMX_INT64;
+    const int8_t *row[16];
+    int at = 0;
+    for (int32_t i = 0; i < count; ++i)
+      for (int32_t r = 0; r < rows[i]; ++r)
+        row[at++] = static_cast<const int8_t *>(requests[i]) + static_cast<int64_t>(r) * k;
+    launch_request_rows(g, row, staging, st);
+    return check_launch("request_rows");
+  }
+  const int64_t row_bytes = static_cast<int64_t>(k) * static_cast<int64_t>(dtype_size(a_dtype));
+  int64_t at = 0;
+  for (int32_t i0 = 0; i0 < count; i0 += kGatherMost) {
+    GatherArgs a{};
+    a.to = staging;
+    const int32_t here = std::min(kGatherMost, count - i0);
+    int64_t most = 0;
+    for (int32_t i = 0; i < here; ++i) {
+      a.from[i] = static_cast<const int8_t *>(requests[i0 + i]);
+      a.at[i] = at;
+      at += rows[i0 + i] * row_bytes;
+      a.at[i + 1] = at;
+      most = std::max(most, at - a.at[i]);
+    }
+    const dim3 grid(static_cast<unsigned>((most + 4095) / 4096), static_cast<unsigned>(here));
+    hipLaunchKernelGGL(gather_requests_kernel, grid, dim3(256), 0, st, a);
+    if (int32_t rc = check_launch("gather_requests")) return rc;
+  }
+  return run_prepared(staging_dev, a_dtype, static_cast<int32_t>(m), k, n, packed_dev, mods, nullptr, 0, nullptr, nullptr,
+                      nullptr, workspace_dev, workspace_bytes, out_dev, stream, packed_form != 0);
+}
+
 // Workspace of rnsmx_matmul_wide: that of the prepared-weight product, then the
 // encoded weight.
 static int64_t wide_weight_at(int64_t m, int64_t k, int64_t n, int32_t channels) {

@@ -1,5 +1,6 @@
-// RNSLinear.forward at decode in one launch: a few rows of float activations
-// are quantized inside the weight-streaming product.
+// Decode in one launch: a few rows of float activations quantized inside the
+// weight-streaming product (RNSLinear.forward), and a few requests' rows read
+// where they lie (continuous batching).
 #include "rnsmx_gemm.hpp"
 #include "rnsmx_quant.hpp"
 
@@ -177,6 +178,132 @@ static void launch_linear_t(const LinearRowsArgs &a, hipStream_t st) {
     hipLaunchKernelGGL((linear_rows_kernel<T, true>), grid, block, lds, st, a);
   else
     hipLaunchKernelGGL((linear_rows_kernel<T, false>), grid, block, lds, st, a);
+}
+
+// ---------------------------------------------------------------------------
+// Continuous batching: the rows of several requests (int8, up to 16 rows in
+// all) against one prepared weight, each row read through its own pointer, so
+// nothing is concatenated first.  Workgroups and waves as above; A fragments
+// come straight from the rows with the weight loads of their chunk.  The rows
+// are also copied to the staging buffer (a row per workgroup), which a caller
+// finds filled as after a concatenation.
+// 4 requests of 1 row, 768 x 768: 4.7 us of a call's 19 were the concatenation.
+// ---------------------------------------------------------------------------
+struct RequestRowsArgs {
+  GemmArgsK<4> g;
+  const int8_t *row[kLinearRowsMax];
+  int8_t *staging;  // [m][K]
+};
+
+template <bool NT>
+__global__ __launch_bounds__(256) void request_rows_kernel(const RequestRowsArgs args) {
+  constexpr int RCAP = 4, U = 4;
+  KArgs<RCAP> &g = kernel_args<GemmArgsK<RCAP>>();
+  RNSMX_KARG(RequestRowsArgs) &all = kernel_args<RequestRowsArgs>();
+  prefetch_kernel_args<static_cast<int>(sizeof(RequestRowsArgs))>();
+  __shared__ int32_t sums[RCAP][256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nthreads = g.threads, ks_n = nthreads >> 6;
+  const int n0 = blockIdx.x * 16, nk = g.kp >> 6, a_k = g.a_k, m = g.m;
+  const int8_t *bp = g.b + static_cast<int64_t>(blockIdx.x) * g.b_ld + lane * 16;
+  const int64_t b_cs = g.b_cs;
+  const int mine = min(lane & 15, m - 1);
+  const int8_t *ap = all.row[0];
+  static_for<kLinearRowsMax - 1>([&](auto I) {
+    constexpr int i = decltype(I)::value + 1;
+    if (mine == i) ap = all.row[i];
+  });
+  const int kofs = (lane >> 4) * 16;
+
+  i32x4 fa[2][U], fb[2][U][RCAP];
+  auto load_chunk = [&](auto BUF, int q) {
+    static_for<U>([&](auto UU) {
+      constexpr int buf = decltype(BUF)::value, u = decltype(UU)::value;
+      const int ks = min(q + u, nk - 1);
+      const int ka = ks * 64 + kofs;
+      fa[buf][u] = load16(ap + min(ka, a_k - 16));  // past K: zeroed at its use
+      static_for<RCAP>([&](auto C) {
+        const int8_t *p = bp + decltype(C)::value * b_cs + ks * 1024;
+        fb[buf][u][decltype(C)::value] = NT ? load16_nt(p) : load16(p);
+      });
+    });
+  };
+  constexpr std::integral_constant<int, 0> b0{};
+  constexpr std::integral_constant<int, 1> b1{};
+  int q = wave * U;
+  const int stride = ks_n * U;
+  load_chunk(b0, q);
+  for (int i = tid; i < RCAP * 256; i += nthreads) (&sums[0][0])[i] = 0;
+  for (int r = blockIdx.x; r < m; r += gridDim.x) {
+    const int8_t *from = all.row[0];
+    static_for<kLinearRowsMax - 1>([&](auto I) {
+      constexpr int i = decltype(I)::value + 1;
+      if (r == i) from = all.row[i];
+    });
+    int8_t *to = all.staging + static_cast<int64_t>(r) * a_k;
+    for (int i = tid * 16; i < a_k; i += nthreads * 16) *reinterpret_cast<i32x4 *>(to + i) = load16(from + i);
+  }
+  Epi<RCAP> e;
+  load_epi<RCAP>(g, e, g.mods.channels);
+  const int n_lim = g.n;
+  i32x4 acc[RCAP];
+  static_for<RCAP>([&](auto C) { acc[decltype(C)::value] = acc_zero(); });
+  auto mfma_chunk = [&](auto BUF, int at) {
+    static_for<U>([&](auto UU) {
+      constexpr int buf = decltype(BUF)::value, u = decltype(UU)::value;
+      if (at + u >= nk) return;
+      const i32x4 a = select16((at + u) * 64 + kofs < a_k, fa[buf][u]);
+      static_for<RCAP>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        acc[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, fb[buf][u][c], acc[c], 0, 0, 0);
+      });
+    });
+  };
+  while (q < nk) {
+    if (q + stride < nk) load_chunk(b1, q + stride);
+    mfma_chunk(b0, q);
+    q += stride;
+    if (q >= nk) break;
+    if (q + stride < nk) load_chunk(b0, q + stride);
+    mfma_chunk(b1, q);
+    q += stride;
+  }
+  __syncthreads();
+  static_for<RCAP>([&](auto C) {
+    static_for<4>([&](auto TT) {
+      constexpr int c = decltype(C)::value, t = decltype(TT)::value;
+      const int r = 4 * (lane >> 4) + t;
+      if (r < m) atomicAdd(&sums[c][r * 16 + (lane & 15)], acc[c][t]);
+    });
+  });
+  __syncthreads();
+  for (int at = tid; at < m * 16; at += nthreads) {
+    const int col = n0 + (at & 15);
+    if (col >= n_lim) continue;
+    int32_t sum[RCAP];
+    static_for<RCAP>([&](auto C) { sum[decltype(C)::value] = sums[decltype(C)::value][at]; });
+    store_value<RCAP, kOutInt64>(e, frac_int<RCAP>(frac_sum<RCAP>(e, sum)),
+                                 static_cast<int64_t>(at >> 4) * e.out_ld + col, ColScale{0.0f, 0.0f});
+  }
+}
+
+bool request_rows_fits(int64_t rows, int64_t k, const rnsmx_moduli_t &mods, int32_t a_dtype) {
+  return a_dtype == RNSMX_INT8 && mods.channels == 4 && rows >= 1 && rows <= kLinearRowsMax && k % 16 == 0 &&
+         raw_accumulator_fits(mods, k);
+}
+
+void launch_request_rows(const GemmArgs &g, const int8_t *const *row, int8_t *staging, hipStream_t st) {
+  RequestRowsArgs a{};
+  a.g = compact_args<4>(g);
+  for (int i = 0; i < kLinearRowsMax; ++i) a.row[i] = row[i < g.m ? i : 0];
+  a.staging = staging;
+  const int chunks = (g.kp / 64 + 3) / 4;
+  a.g.threads = 64 * (chunks < 4 ? 3 : 4);
+  const dim3 grid(static_cast<unsigned>((g.n + 15) / 16)), block(static_cast<unsigned>(a.g.threads));
+  if (g.kp >= 4096)
+    hipLaunchKernelGGL(request_rows_kernel<true>, grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL(request_rows_kernel<false>, grid, block, 0, st, a);
 }
 
 bool linear_rows_fits(int64_t rows, int64_t k, const rnsmx_moduli_t &mods, int32_t quant_bits, bool adaptive) {

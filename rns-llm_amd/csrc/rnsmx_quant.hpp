@@ -88,4 +88,9 @@ __device__ __forceinline__ float quant_value(float v, float s, float qmax) {
 bool linear_rows_fits(int64_t rows, int64_t k, const rnsmx_moduli_t &mods, int32_t quant_bits, bool adaptive);
 void launch_linear_rows(const GemmArgs &g, const QuantArgs &q, int32_t x_dtype, hipStream_t st);
 
+// Requests of a few int8 rows in one launch (rnsmx_linear.hip): row[i] the
+// 16-byte aligned row i < g.m, copied to staging [m][K] too.
+bool request_rows_fits(int64_t rows, int64_t k, const rnsmx_moduli_t &mods, int32_t a_dtype);
+void launch_request_rows(const GemmArgs &g, const int8_t *const *row, int8_t *staging, hipStream_t st);
+
 }  // namespace rnsmx

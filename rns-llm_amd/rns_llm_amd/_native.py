@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "rnsmx_prepare_weight",
     "rnsmx_prepared_workspace_bytes",
     "rnsmx_matmul_prepared_fused",
+    "rnsmx_matmul_requests",
     "rnsmx_wide_workspace_bytes",
     "rnsmx_matmul_wide",
     "rnsmx_matmul_prepared_fused_noalloc",
@@ -141,6 +142,8 @@ _SIGNATURES = {
         _I32, [_P, _I32, _I32, _I32, _I32, _P, ctypes.POINTER(Moduli), _P, _I32,
                ctypes.POINTER(Adaptive), ctypes.POINTER(Epilogue), ctypes.POINTER(Plan),
                _P, _I64, _P, _P]),
+    "rnsmx_matmul_requests": (
+        _I32, [_P, _P, _I32, _I32, _I32, _I32, _P, ctypes.POINTER(Moduli), _I32, _P, _P, _I64, _P, _P]),
     "rnsmx_wide_workspace_bytes": (_I64, [_I64, _I64, _I64, _I32]),
     "rnsmx_matmul_wide": (_I32, [_P, _P, _I32, _I32, _I32, _I32, ctypes.POINTER(Moduli), _P, _I64, _P, _P]),
     "rnsmx_matmul_prepared_fused_noalloc": (

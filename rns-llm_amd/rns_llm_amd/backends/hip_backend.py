@@ -27,7 +27,6 @@ from __future__ import annotations
 
 import ctypes
 import functools
-import itertools
 from collections import Counter
 from collections.abc import Mapping
 from dataclasses import dataclass, field
@@ -965,30 +964,63 @@ class HipRNSBackend:
         if len(requests) == 0:
             raise ValueError("no requests to batch")
         for index, request in enumerate(requests):
-            self._validate_matrix(request, f"request {index}", 2)
-        kinds = {(r.dtype, r.device) for r in requests}
-        if len(kinds) != 1:
-            raise ValueError(f"requests mix dtypes/devices: {sorted(map(str, kinds))}")
-        widths = {int(r.shape[1]) for r in requests}
-        if widths != {prepared_weight.k}:
-            raise ValueError(f"request widths {sorted(widths)} differ from the weight's K = {prepared_weight.k}")
-        rows = tuple(int(r.shape[0]) for r in requests)
+            if not (request.is_cuda and request.ndim == 2 and request.is_contiguous()):
+                self._validate_matrix(request, f"request {index}", 2)
+        first = requests[0]
+        dtype, device, k = first.dtype, first.device, prepared_weight.k
+        shapes = [r.shape for r in requests]
+        if any(r.dtype != dtype or r.device != device for r in requests):
+            raise ValueError("requests mix dtypes/devices: "
+                             f"{sorted(map(str, {(r.dtype, r.device) for r in requests}))}")
+        if any(s[1] != k for s in shapes):
+            raise ValueError(f"request widths {sorted({int(s[1]) for s in shapes})} differ from the weight's K = {k}")
+        rows = tuple([int(s[0]) for s in shapes])
         if workspace is None:
-            (dtype, device), = kinds
             workspace = self.create_request_batch_workspace(
-                device=device, dtype=dtype, rows_per_request=rows, k=prepared_weight.k,
+                device=device, dtype=dtype, rows_per_request=rows, k=k,
                 channels=len(prepared_weight.moduli), n=prepared_weight.n)
-        if workspace.rows_per_request != rows or workspace.k != prepared_weight.k:
+        if workspace.rows_per_request != rows or workspace.k != k:
             raise ValueError(f"batch workspace holds rows {workspace.rows_per_request} x K={workspace.k}, "
-                             f"requests are {rows} x K={prepared_weight.k}")
-        torch.cat(tuple(requests), dim=0, out=workspace.activations)
-        merged = self.matmul_prepared_fused(workspace.activations, prepared_weight,
-                                            lut_channels=lut_channels, workspace=workspace.fused)
-        bounds = list(itertools.accumulate(rows, initial=0))
-        views = tuple(merged[lo:hi] for lo, hi in zip(bounds, bounds[1:]))
+                             f"requests are {rows} x K={k}")
+        merged = self._merged_product(requests, rows, prepared_weight, lut_channels, workspace)
+        if merged is None:
+            torch.cat(tuple(requests), dim=0, out=workspace.activations)
+            merged = self.matmul_prepared_fused(workspace.activations, prepared_weight,
+                                                lut_channels=lut_channels, workspace=workspace.fused)
+        views = merged.split(rows)
         self._stats["continuous_batch_calls"] += 1
         self._stats["continuous_batch_requests"] += len(rows)
         return tuple(v.clone() for v in views) if clone_outputs else views
+
+    def _merged_product(self, requests, rows: tuple[int, ...], prepared: PreparedRNSWeight, lut_channels: int,
+                        workspace: RNSRequestBatchWorkspace) -> torch.Tensor | None:
+        """The requests' product and the filled staging buffer in one library
+        call; None where the buffer is not the requests' own kind, or the
+        product's checks have to refuse the call."""
+        staging, fused = workspace.activations, workspace.fused
+        device, dtype, m = staging.device, staging.dtype, sum(rows)
+        n, channels = prepared.n, len(prepared.moduli)
+        if (dtype != requests[0].dtype or dtype not in _DTYPE_MAX_ABS or device != requests[0].device
+                or device != prepared.packed.device or tuple(staging.shape) != (m, prepared.k)
+                or not staging.is_contiguous() or staging.data_ptr() % 16 or lut_channels not in (0, 1, 2)
+                or lut_channels > channels or n == 0):
+            return None
+        self._check_workspace(fused, channels=channels, m=m, n=n, device=device)
+        packed_form = prepared.form == "packed"
+        scratch = self._scratch(fused, self._packed_workspace_bytes(m, prepared.k, n, channels, None) if packed_form
+                                else self._prepared_workspace_bytes(m, prepared.k, n, channels, None))
+        stats = self._stats
+        stats["encode_centered_calls"] += 1
+        stats["encode_centered_values"] += m * prepared.k
+        stats["fused_gemm_calls"] += 1
+        stats[f"fused_gemm_channels_{channels}"] += 1
+        count = len(rows)
+        _native.check(self._lib.rnsmx_matmul_requests(
+            (ctypes.c_void_p * count)(*[r.data_ptr() for r in requests]), (ctypes.c_int32 * count)(*rows), count,
+            _native.dtype_code(dtype), prepared.k, n, prepared.packed.data_ptr(),
+            self._constants(device, prepared.moduli).native_ref, packed_form, staging.data_ptr(), scratch.data_ptr(),
+            scratch.numel(), fused.output.data_ptr(), _stream_handle(device)))
+        return fused.output
 
     # ------------------------------------------------------------------
     # Convenience wrappers (cuda_backend.py:733-799): both integer operands

@@ -1,0 +1,59 @@
+"""Continuous batching in one library call: up to 16 int8 rows read where they
+lie, other batches gathered first; requests off a 16-byte boundary, K that
+fills no step or no fragment, more requests than one gather launch takes,
+packed weights.  Outputs are each request's exact product, the staging buffer
+holds the concatenation, and the workspace serves the next call."""
+import pytest
+import torch
+
+from oracle import rns_oracle as ro
+
+pytestmark = pytest.mark.gpu
+
+DENSE4 = (255, 253, 251, 247)
+DENSE6 = DENSE4 + (241, 239)
+
+
+def exact(a, w_nk):
+    return torch.from_numpy(ro.exact_matmul(a.cpu().numpy(), w_nk.t().numpy()))
+
+
+@pytest.mark.parametrize("rows", [(1,), (1, 1, 1, 1), (3, 1, 12), (16,), (8, 9), (5, 40, 1), (1,) * 35, (2,) * 8])
+@pytest.mark.parametrize("k,n", [(768, 100), (80, 17), (777, 64), (4096, 48), (1040, 7)])
+@pytest.mark.parametrize("dtype,packed", [(torch.int8, False), (torch.int16, False), (torch.int16, True), (torch.int32, False)])
+def test_merged_products(backend, rows, k, n, dtype, packed):
+    gen = torch.Generator().manual_seed(sum(rows) + k)
+    lim = 127 if dtype == torch.int8 else 2047
+    moduli = DENSE4 if dtype == torch.int8 else DENSE6
+    w = torch.randint(-lim, lim + 1, (n, k), generator=gen, dtype=torch.int32).to(torch.int8 if lim == 127 else torch.int16)
+    prepared = (backend.prepare_weight_packed_nk if packed else backend.prepare_weight_nk)(w.cuda(), moduli)
+    ws = backend.create_request_batch_workspace(device=torch.device("cuda"), dtype=dtype, rows_per_request=rows, k=k,
+                                                channels=len(moduli), n=n)
+    for shift in (0, 1):  # the second time every request starts off a 16-byte boundary
+        requests = []
+        for r in rows:
+            t = torch.empty((r * k + shift,), dtype=dtype, device="cuda")[shift:].view(r, k)
+            requests.append(t.copy_(torch.randint(-lim - 1, lim + 1, (r, k), generator=gen, dtype=torch.int32)))
+        backend.reset_stats()
+        outs = backend.matmul_prepared_fused_requests(requests, prepared, workspace=ws)
+        assert backend.stats_snapshot() == {
+            "encode_centered_calls": 1, "encode_centered_values": sum(rows) * k, "fused_gemm_calls": 1,
+            f"fused_gemm_channels_{len(moduli)}": 1, "continuous_batch_calls": 1, "continuous_batch_requests": len(rows)}
+        assert torch.equal(ws.activations, torch.cat(requests))
+        assert len(outs) == len(rows) and outs[0].data_ptr() == ws.fused.output.data_ptr()
+        for request, out in zip(requests, outs):
+            assert torch.equal(out.cpu(), exact(request, w))
+    clones = backend.matmul_prepared_fused_requests(requests, prepared, clone_outputs=True)
+    assert torch.equal(torch.cat(clones), ws.fused.output)
+
+
+def test_refusals(backend):
+    w = torch.ones((16, 64), dtype=torch.int8).cuda()
+    prepared = backend.prepare_weight_nk(w, DENSE4)
+    x = torch.ones((2, 64), dtype=torch.int8).cuda()
+    ws = backend.create_request_batch_workspace(device=x.device, dtype=torch.int8, rows_per_request=(2,), k=64,
+                                                channels=4, n=16)
+    for requests, kw in (([], {}), ([x, x.to(torch.int16)], {}), ([x[:, :32].contiguous()], {}), ([x.t()], {}), ([x, x], {"workspace": ws}),
+                         ([x], {"lut_channels": 3}), ([x.float()], {}), ([x.cpu()], {})):
+        with pytest.raises(ValueError):
+            backend.matmul_prepared_fused_requests(requests, prepared, **kw)
