@@ -171,6 +171,7 @@ inline GemmArgsK<RCAP> compact_args(const GemmArgs &g) {
 // kLdsWide: the LDS-staged kernel with 256 x 96 tiles (lds_wide_kernel).
 // kBytesRows, kBytesLds: packed weights by byte products (rnsmx_bytes.hpp):
 // decode (mb fragments of tokens), tiles of 16 mb rows.
+// kUnits: residue planes by channel units (rnsmx_units.hip), 32 mb x 64 nb.
 enum GemmKind {
   kAuto = 0,
   kStream = 1,
@@ -182,7 +183,8 @@ enum GemmKind {
   kLdsWide = 7,
   kLdsPlanes = 8,
   kBytesRows = 9,
-  kBytesLds = 10
+  kBytesLds = 10,
+  kUnits = 11
 };
 
 // ks: waves splitting K (stream kernel) or ring depth, 0 = automatic (MFMA
@@ -229,6 +231,8 @@ RNSMX_GEMM_PARTS_DECL(10)
 // The byte-product kernels (rnsmx_bytes.hip), ab bytes per activation; false
 // when there is none for the choice.
 bool launch_bytes(const GemmArgs &g, int ab, const GemmChoice &c, hipStream_t st);
+// Residue planes by channel units (rnsmx_units.hip), up to 6 channels.
+bool launch_units(const GemmArgs &g, const GemmChoice &c, hipStream_t st);
 
 // Kernel arguments read in place from the kernarg segment (constant address
 // space, scalar loads).  A by-value struct parameter used as an ordinary
@@ -3019,6 +3023,10 @@ inline GemmGrid gemm_grid(const GemmChoice &c, int64_t m, int64_t n) {
     r.tiles = cdiv(m, kLdsBM) * cdiv(n, bn);
     r.waves = 8;
     r.chunks = (kLdsBM / 16 / 4) * (bn / 16 / 2);
+  } else if (c.kind == kUnits) {
+    r.tiles = cdiv(m, 32 * c.mb) * cdiv(n, 64 * c.nb);
+    r.waves = 8;
+    r.chunks = c.mb * c.nb;  // words of 256 bytes per wave and channel
   } else if (c.kind == kBytesRows) {
     r.tiles = cdiv(n, 16);
     r.waves = c.ks;

@@ -1028,7 +1028,7 @@ static bool split_fits(const GemmChoice &c, const GemmArgs &g) {
     built = stream_splits(rcap, c.mb, c.nb) && c.ks == 1;
   else if (c.kind == kLdsPlanes)
     built = rcap == 4 || rcap == 6;
-  else if (c.kind == kBytesLds)
+  else if (c.kind == kBytesLds || c.kind == kUnits)
     built = true;
   else if (is_lds(c.kind))
     built = rcap <= 4;
@@ -1039,6 +1039,10 @@ static bool split_fits(const GemmChoice &c, const GemmArgs &g) {
 
 // Exchange-area bytes of a choice (0 without a split).
 static int64_t xchg_bytes(const GemmChoice &c, const GemmArgs &g) {
+  if (c.kind == kUnits) {  // a byte per channel and element of every tile
+    const GemmGrid gr = gemm_grid(c, g.m, g.n);
+    return gr.tiles * gr.waves * g.mods.channels * gr.chunks * 256;
+  }
   if (c.splits <= 1) return 0;
   int splits, kchunk;
   split_steps(c, g.kp / 64, splits, kchunk);
@@ -1123,18 +1127,92 @@ static GemmChoice auto_plan(const GemmArgs &g, bool araw, bool allow_split) {
   return c;
 }
 
+// Residue planes by channel units (rnsmx_units.hip): 5 or 6 channels, where a
+// wave that holds every channel has registers for a small tile only; rows
+// addressed by 32-bit offsets within a plane; a counter per (tile, wave).
+static bool units_fit(const GemmChoice &c, const GemmArgs &g, bool araw) {
+  const GemmGrid gr = gemm_grid(c, g.m, g.n);
+  return !araw && (g.mods.channels == 5 || g.mods.channels == 6) &&
+         static_cast<int64_t>(g.m) * g.a_ld < (int64_t{1} << 32) - 256 &&
+         gr.tiles * gr.waves <= RNSMX_SPLIT_TICKETS;
+}
+
+// Whether an automatic plan takes channel units instead of `other`: by the
+// estimated times of both in microseconds, linear in the K steps, with
+// constants fitted to 5- and 6-channel products from 17 to 1300 rows, K 512 to
+// 4096, N 512 to 12288.  A unit's K step is short (one channel), so units win
+// where the other plan leaves CUs idle or runs a few long rounds: at
+// 128 x 4096 x 4096 in 6 channels 32 us against 49, 640 x 2048 x 2048 36
+// against 66, 77 x 1531 x 1000 in 5 15.0 against 18.4.  They lose when their
+// workgroups exceed four per CU (the residues they exchange then cost more
+// than the shorter steps save: 512 x 5120 x 2048 55 us against 46) and below
+// 17 rows, where the streaming kernels read the weight as fast.  The 5 %
+// between the estimates covers their error: over 180 shapes no product that
+// took units was slower by more than the timing's 2 %.
+static bool units_auto(const GemmArgs &g, const GemmChoice &other, GemmChoice &c) {
+  if (g.m <= 16) return false;
+  auto rounds = [](int64_t workgroups) { return static_cast<double>((workgroups + 255) / 256); };
+  const double steps = g.kp / 64, channels = g.mods.channels / 6.0;
+  const int64_t tiles = gemm_grid(other, g.m, g.n).tiles;
+  double before;
+  if (other.kind == kMfma) {
+    before = 7 + 0.35 * other.mb * other.nb * steps * channels * rounds(tiles);
+  } else if (other.kind == kLdsPlanes) {
+    // a tail split shortens the last round, a uniform one the only round
+    const double r = other.splits <= 1 ? rounds(tiles)
+                     : other.tail      ? static_cast<double>((tiles - 1) / 256) + 1.0 / other.splits
+                                       : 1.0 / other.splits;
+    before = 8 + 1.2 * steps * r + (tiles <= 256 ? 5 * (other.splits - 1) : 0);
+  } else if (other.kind == kStream) {
+    before = 7 + 0.22 * steps * channels * rounds(tiles);
+  } else {
+    return false;
+  }
+  // base and K step by workgroups per CU
+  static constexpr struct {
+    int mb, nb;
+    double base[4], step[4];
+  } units[2] = {{2, 1, {8.5, 10, 11.5, 13}, {0.3, 0.3, 0.38, 0.58}},
+                {4, 2, {16.5, 20, 24, 28}, {0.3, 0.36, 0.75, 0.8}}};
+  double best = 0.95 * before;
+  bool found = false;
+  for (const auto &u : units) {
+    const GemmChoice t{kUnits, u.mb, u.nb, 0, 1, 0};
+    const int64_t per_cu = (gemm_grid(t, g.m, g.n).tiles * g.mods.channels + 255) / 256;
+    if (per_cu > 4 || !units_fit(t, g, false)) continue;
+    const double now = u.base[per_cu - 1] + u.step[per_cu - 1] * steps;
+    if (now < best) {
+      best = now;
+      c = t;
+      found = true;
+    }
+  }
+  return found;
+}
+
+// units: the caller has a workspace with an exchange area, so an automatic plan
+// for residue planes may take channel units.
 static int32_t plan_from(const rnsmx_plan_t *plan, const GemmArgs &g, bool araw, bool allow_split,
-                         GemmChoice &c) {
+                         GemmChoice &c, bool units = false) {
   if (plan == nullptr || plan->kind == kAuto) {
     c = auto_plan(g, araw, allow_split);
+    GemmChoice by_channel{};
+    if (units && !araw && units_auto(g, c, by_channel)) c = by_channel;
     return RNSMX_OK;
   }
   const int k = plan->kind;
+  if (k == kUnits) {
+    c = GemmChoice{k, plan->mb, plan->nb, 0, 1, 0};
+    const bool built = (c.mb == 4 && c.nb == 2) || (c.mb == 2 && c.nb == 1);
+    if (!units || !built || !units_fit(c, g, araw))
+      return fail(RNSMX_EINVAL, "channel-unit plans take residue planes of 5 or 6 channels in a workspace, tiles 4 x 2 or 2 x 1");
+    return RNSMX_OK;
+  }
   if (k != kStream && k != kMfma && k != kLds && k != kStreamWide && k != kMfma3 && k != kLdsWide &&
       k != kLdsPlanes)
     return fail(RNSMX_EINVAL,
                 "plan kind must be 0 (auto), 1 (stream), 2 (mfma), 3 (lds), 4 (wide stream), 5 (3-wave mfma), "
-                "7 (wide lds) or 8 (residue-plane lds)");
+                "7 (wide lds), 8 (residue-plane lds) or 11 (channel units)");
   if (!is_lds(k) && (plan->mb < 1 || plan->nb < 1)) return fail(RNSMX_EINVAL, "tile blocks must be positive");
   c = GemmChoice{k, plan->mb, plan->nb, plan->ks, std::max(1, plan->splits), plan->tail != 0};
   if (c.splits > 1 && (!allow_split || !split_fits(c, g)))
@@ -1179,6 +1257,13 @@ static int32_t launch_gemm(GemmArgs g, bool araw, const GemmChoice &c, uint32_t 
       return RNSMX_EINVAL;
     }
     return check_launch("gemm_bytes");
+  }
+  if (c.kind == kUnits) {
+    if (tickets == nullptr || xchg == nullptr || !launch_units(g, c, st)) {
+      set_error("no channel-unit kernel for tile %d x %d", c.mb, c.nb);
+      return RNSMX_EINVAL;
+    }
+    return check_launch("gemm_units");
   }
   using PartFn = bool (*)(const GemmArgs &, bool, const GemmChoice &, hipStream_t);
 #define RNSMX_PARTS(R)                                                                      \
@@ -1753,12 +1838,12 @@ static PreparedLayout packed_layout(int64_t m, int64_t kp, int32_t channels, int
 // Workspace bytes of one prepared-path call shape and plan, for A read in
 // place (araw) or as residue planes.
 static int64_t prepared_need(bool araw, int64_t m, int64_t k, int64_t n, int32_t channels,
-                             const rnsmx_plan_t *plan) {
+                             const rnsmx_plan_t *plan, bool units = true) {
   int64_t xchg = 0;
   if (m > 0 && n > 0) {
     const GemmArgs g = plan_args(m, n, k, channels, araw);
     GemmChoice c{};
-    if (plan_from(plan, g, araw, true, c) == RNSMX_OK) xchg = xchg_bytes(c, g);
+    if (plan_from(plan, g, araw, true, c, units) == RNSMX_OK) xchg = xchg_bytes(c, g);
   }
   return prepared_layout(araw, m, k, channels, xchg).total;
 }
@@ -1826,7 +1911,10 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   GemmArgs g = plan_args(m, n, k, R, araw);
   g.mods = *mods;
   GemmChoice c{};
-  if (int32_t rc = packed ? packed_plan_from(plan, g, c, a_dtype) : plan_from(plan, g, araw, true, c)) return rc;
+  if (int32_t rc = packed ? packed_plan_from(plan, g, c, a_dtype) : plan_from(plan, g, araw, true, c, true)) return rc;
+  if (c.kind == kUnits && (plan == nullptr || plan->kind == kAuto) &&
+      workspace_bytes < prepared_layout(araw, m, k, R, xchg_bytes(c, g)).total)
+    c = auto_plan(g, araw, true);  // a workspace made for more rows may hold no exchange area
   const bool bytes = c.kind == kBytesRows || c.kind == kBytesLds;
   const PreparedLayout l = packed ? packed_layout(m, kp, R, xchg_bytes(c, g))
                                   : prepared_layout(araw, m, k, R, xchg_bytes(c, g));
@@ -2072,9 +2160,12 @@ int32_t rnsmx_matmul_wide(const void *a_dev, const void *b_dev, int32_t dtype, i
   // encoder, so the workspace may hold anything before the call
   const bool araw = raw_route(dtype, k, *mods, nullptr);
   const GemmArgs g = plan_args(m, n, k, mods->channels, araw);
-  const GemmChoice c = auto_plan(g, araw, true);
+  GemmChoice c{};
+  if (int32_t rc = plan_from(nullptr, g, araw, true, c, true)) return rc;
   const GemmGrid gr = gemm_grid(c, m, n);
-  const int64_t ntickets = c.splits > 1 ? (gr.tiles - whole_tiles(c, gr.tiles)) * gr.waves : 0;
+  const int64_t ntickets = c.kind == kUnits ? gr.tiles * gr.waves
+                           : c.splits > 1   ? (gr.tiles - whole_tiles(c, gr.tiles)) * gr.waves
+                                            : 0;
   const int64_t kp = round_up(k, RNSMX_K_ALIGN), n16 = (static_cast<int64_t>(n) + 15) / 16;
   EncodeArgs e{};
   e.values = b_dev;
@@ -2191,6 +2282,11 @@ int32_t rnsmx_matmul_prepared_fused_noalloc(const void *a_dev, int32_t a_dtype, 
     own = rnsmx_plan_t{c.kind, c.mb, c.nb, c.ks, 1, 0};
     run_plan = &own;
     need = prepared_layout(raw, m, k, mods->channels, 0).total;
+  } else if (!araw && (plan == nullptr || plan->kind == kAuto)) {
+    // named, so that the workspace entry point does not take channel units,
+    // whose exchange area this scratch is not sized for
+    own = rnsmx_plan_t{c.kind, c.mb, c.nb, c.ks, c.splits, c.tail};
+    run_plan = &own;
   }
   if (need > RNSMX_NOALLOC_SCRATCH_BYTES) {
     set_error("this call needs %lld bytes of scratch; the static scratch holds %lld (use "
@@ -2351,9 +2447,14 @@ struct LinearLayout {
   int64_t gemm, quant, scale, q, total;
 };
 
-static LinearLayout linear_layout(int64_t rows, int64_t k, int64_t n, int32_t channels, int32_t quant_bits) {
+// units: with room for the exchange of channel units.
+static LinearLayout linear_layout(int64_t rows, int64_t k, int64_t n, int32_t channels, int32_t quant_bits,
+                                  bool units = true) {
   LinearLayout l{};
   l.gemm = rnsmx_prepared_workspace_bytes(rows, k, n, channels, nullptr);
+  if (l.gemm >= 0 && !units)
+    l.gemm = std::max(prepared_need(true, rows, k, n, channels, nullptr, false),
+                      prepared_need(false, rows, k, n, channels, nullptr, false));
   if (l.gemm < 0) {
     l.total = -1;
     return l;
@@ -2382,8 +2483,9 @@ int32_t rnsmx_linear_forward(const void *x_dev, int32_t x_dtype, int32_t rows, i
   if (!mods || mods->channels < 1) return fail(RNSMX_EINVAL, "moduli are not initialised");
   if (rows < 0 || k < 1 || n < 0) return fail(RNSMX_EINVAL, "bad linear shape");
   if (!w_scale_dev) return fail(RNSMX_EINVAL, "the weight scales are missing");
-  const LinearLayout l = linear_layout(rows, k, n, mods->channels, quant_bits);
+  LinearLayout l = linear_layout(rows, k, n, mods->channels, quant_bits);
   if (l.total < 0) return fail(RNSMX_EINVAL, "bad linear shape");
+  if (workspace_bytes < l.total) l = linear_layout(rows, k, n, mods->channels, quant_bits, false);
   if (!workspace_dev) return fail(RNSMX_EINVAL, "null workspace");
   if (workspace_bytes < l.total) {
     set_error("workspace too small: %lld < %lld bytes", static_cast<long long>(workspace_bytes),

@@ -21,7 +21,7 @@ GEMM_CAPACITIES = (3, 4, 6, 10)
 GEMM_PARTS = 6
 # (source, object name, extra flags)
 UNITS = [("rnsmx_kernels.hip", "rnsmx_kernels", []), ("rnsmx_bytes.hip", "rnsmx_bytes", []),
-         ("rnsmx_linear.hip", "rnsmx_linear", []),
+         ("rnsmx_linear.hip", "rnsmx_linear", []), ("rnsmx_units.hip", "rnsmx_units", []),
          ("rnsmx_host.cpp", "rnsmx_host", [])] + [
     ("rnsmx_gemm_part.hip", f"rnsmx_gemm_r{r}_p{p}", [f"-DRNSMX_RCAP={r}", f"-DRNSMX_PART={p}"])
     for r in GEMM_CAPACITIES for p in range(GEMM_PARTS)]
