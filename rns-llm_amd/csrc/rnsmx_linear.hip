@@ -306,9 +306,21 @@ void launch_request_rows(const GemmArgs &g, const int8_t *const *row, int8_t *st
     hipLaunchKernelGGL(request_rows_kernel<false>, grid, block, 0, st, a);
 }
 
-bool linear_rows_fits(int64_t rows, int64_t k, const rnsmx_moduli_t &mods, int32_t quant_bits, bool adaptive) {
-  return quant_bits == 8 && !adaptive && mods.channels == 4 && rows >= 1 && rows <= kLinearRowsMax &&
-         rows * k <= kLinearRowsValues && raw_accumulator_fits(mods, k);
+// Every workgroup quantizes all M K values, so the launches saved pay for M K N
+// up to a line: against the quantizer's kernels and the product, float16
+// (device time), 4 x 768 x 8192 9.6 -> 9.2 us but 8 x 768 x 4571 8.0 -> 8.4;
+// from K = 1024, where those spend longer, 4 x 2048 x 4571 14.0 -> 11.3 but
+// 8 x 1024 x 8192 11.8 -> 12.1; N = 12288, 1 row, 768 11.1 -> 11.6.  Values that
+// are not read 16 bytes at a time (K no multiple of 16, or the first off a
+// 16-byte boundary) cost more each: 4 x 1001 x 8192 16.5 -> 14.7 us, 8 x 662 x
+// 2304 10.4 -> 11.3.
+bool linear_rows_fits(int64_t rows, int64_t k, int64_t n, const rnsmx_moduli_t &mods, int32_t quant_bits,
+                      bool adaptive, bool aligned) {
+  if (quant_bits != 8 || adaptive || mods.channels != 4 || rows < 1 || rows > kLinearRowsMax || n < 1 || n > 8192 ||
+      rows * k > kLinearRowsValues || !raw_accumulator_fits(mods, k))
+    return false;
+  if (!aligned || k % 16 != 0) return rows * k <= kLinearRowsValues / 2;
+  return k < 1024 ? rows * k * n <= 24 << 20 : rows * k * n < 64 << 20;
 }
 
 void launch_linear_rows(const GemmArgs &g, const QuantArgs &q, int32_t x_dtype, hipStream_t st) {

@@ -85,7 +85,9 @@ __device__ __forceinline__ float quant_value(float v, float s, float qmax) {
 
 // The decode layer in one launch (rnsmx_linear.hip): whether it serves a call,
 // and its launch (g: shape, weight and epilogue; q: x, vec, qmax, rcp).
-bool linear_rows_fits(int64_t rows, int64_t k, const rnsmx_moduli_t &mods, int32_t quant_bits, bool adaptive);
+// aligned: the activations start on a 16-byte boundary.
+bool linear_rows_fits(int64_t rows, int64_t k, int64_t n, const rnsmx_moduli_t &mods, int32_t quant_bits,
+                      bool adaptive, bool aligned);
 void launch_linear_rows(const GemmArgs &g, const QuantArgs &q, int32_t x_dtype, hipStream_t st);
 
 // Requests of a few int8 rows in one launch (rnsmx_linear.hip): row[i] the

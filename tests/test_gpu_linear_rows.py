@@ -18,7 +18,9 @@ def layer_of(backend, k, n, dtype, bias=True, **kw):
 
 
 @pytest.mark.parametrize("rows,k,n", [(1, 768, 2304), (1, 8192, 48), (2, 4096, 33), (16, 512, 17), (16, 513, 64), (10, 777, 40),
-                                      (13, 600, 31), (3, 1001, 70), (1, 515, 16), (8, 1024, 100), (17, 481, 32), (9, 911, 16)])
+                                      (13, 600, 31), (3, 1001, 70), (1, 515, 16), (8, 1024, 100), (17, 481, 32), (9, 911, 16),
+                                      # both sides of the lines where the quantizer's own kernels take over
+                                      (4, 768, 8192), (4, 768, 8193), (4, 1024, 97), (4, 1025, 97), (5, 777, 97)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bias", [True, False])
 def test_rows_equal_the_float_chain(backend, rows, k, n, dtype, bias):
