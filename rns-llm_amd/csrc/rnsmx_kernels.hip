@@ -1383,8 +1383,11 @@ static GemmChoice packed_auto(const GemmArgs &g) {
 }
 
 // Byte products (rnsmx_bytes.hpp) for int8 (ab = 1) and int16 (ab = 2)
-// activations, K within the int32 sums.
-static bool bytes_fit(const GemmArgs &g) { return g.kp <= kBytesMaxKp; }
+// activations, K within the int32 sums and rows addressed by 32-bit offsets
+// within a plane (bytes_lds_kernel's loads; other products keep the channel form).
+static bool bytes_fit(const GemmArgs &g) {
+  return g.kp <= kBytesMaxKp && static_cast<int64_t>(g.m) * round_up(g.kp, 128) < (int64_t{1} << 32) - 256;
+}
 
 // Kernel, tile and split for byte products, from a sweep on MI355X (int16, K
 // 768-4096, N 768-12288, M 16-4096; us per call, planes launch included).
@@ -1434,7 +1437,7 @@ static int32_t packed_plan_from(const rnsmx_plan_t *plan, const GemmArgs &g, Gem
   }
   if (plan->kind == kBytesRows || plan->kind == kBytesLds) {
     if (a_dtype == RNSMX_INT32 || !bytes_fit(g))
-      return fail(RNSMX_EINVAL, "byte-product plans take int8 or int16 activations and K up to 65472");
+      return fail(RNSMX_EINVAL, "byte-product plans take int8 or int16 activations, K up to 65472 and planes below 4 GiB");
     c = GemmChoice{plan->kind, plan->mb, 1, plan->ks, std::max(1, plan->splits), plan->tail != 0};
     if (c.kind == kBytesRows) {
       const int tokens = plan->mb * (a_dtype == RNSMX_INT8 ? 16 : 8);
