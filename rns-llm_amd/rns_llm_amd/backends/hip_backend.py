@@ -1005,6 +1005,11 @@ class HipRNSBackend:
                 or not staging.is_contiguous() or staging.data_ptr() % 16 or lut_channels not in (0, 1, 2)
                 or lut_channels > channels or n == 0):
             return None
+        pointers = [r.data_ptr() for r in requests]
+        begin = staging.data_ptr()
+        end = begin + staging.nbytes
+        if any(begin - r.nbytes < p < end for p, r in zip(pointers, requests)):
+            return None  # rows inside the buffer they would be copied to
         self._check_workspace(fused, channels=channels, m=m, n=n, device=device)
         packed_form = prepared.form == "packed"
         scratch = self._scratch(fused, self._packed_workspace_bytes(m, prepared.k, n, channels, None) if packed_form
@@ -1016,7 +1021,7 @@ class HipRNSBackend:
         stats[f"fused_gemm_channels_{channels}"] += 1
         count = len(rows)
         _native.check(self._lib.rnsmx_matmul_requests(
-            (ctypes.c_void_p * count)(*[r.data_ptr() for r in requests]), (ctypes.c_int32 * count)(*rows), count,
+            (ctypes.c_void_p * count)(*pointers), (ctypes.c_int32 * count)(*rows), count,
             _native.dtype_code(dtype), prepared.k, n, prepared.packed.data_ptr(),
             self._constants(device, prepared.moduli).native_ref, packed_form, staging.data_ptr(), scratch.data_ptr(),
             scratch.numel(), fused.output.data_ptr(), _stream_handle(device)))

@@ -57,3 +57,15 @@ def test_refusals(backend):
                          ([x], {"lut_channels": 3}), ([x.float()], {}), ([x.cpu()], {})):
         with pytest.raises(ValueError):
             backend.matmul_prepared_fused_requests(requests, prepared, **kw)
+
+
+@pytest.mark.parametrize("rows", [(2, 2), (20, 20)])
+def test_requests_inside_the_staging_buffer_are_refused(backend, rows):
+    """Rows that would be copied over each other: refused, whatever their number."""
+    prepared = backend.prepare_weight_nk(torch.ones((16, 64), dtype=torch.int8).cuda(), DENSE4)
+    ws = backend.create_request_batch_workspace(device=torch.device("cuda"), dtype=torch.int8, rows_per_request=rows,
+                                                k=64, channels=4, n=16)
+    ws.activations.fill_(1)
+    half = rows[0]
+    with pytest.raises(RuntimeError):
+        backend.matmul_prepared_fused_requests([ws.activations[half:], ws.activations[:half]], prepared, workspace=ws)
