@@ -91,7 +91,7 @@ typedef struct rnsmx_moduli {
  * and packed weights; 128 x 128 tiles, 4- or 6-channel capacity, K a
  * multiple of 256; mb, nb, ks ignored; splits and tail as for kind 3), 9 and
  * 10 = packed weights by byte products (int8 and int16 activations, K up to
- * 65472): 9 reads the activations as they are (up to mb = 1, 2 or 4 fragments
+ * 65472, an activation byte plane below 4 GiB): 9 reads the activations as they are (up to mb = 1, 2 or 4 fragments
  * of 8 int16 or 16 int8 tokens, ks waves splitting K, never split), 10 runs
  * tiles of 16*mb x 24*mb (mb 4 or 8), split as kind 3.
  * splits: workgroups splitting K per output tile (0 or 1 = none; up to 4
