@@ -363,8 +363,10 @@ int32_t rnsmx_prepare_weight_packed(const void *b_nk_dev, int32_t dtype,
                                     int32_t *absmax_dev, void *stream);
 
 /* Bytes of workspace rnsmx_matmul_packed_fused needs for an M x N x K
- * product with `channels` moduli under `plan` (NULL: the automatic plan);
- * -1 for a bad shape or a plan the call would reject. */
+ * product with `channels` moduli under `plan` (NULL: the automatic plan),
+ * whatever the activation dtype; -1 for a bad shape or a plan the call would
+ * reject.  In a workspace without room for the split exchange (one made for
+ * more rows need not have it) the automatic byte product runs unsplit. */
 int64_t rnsmx_packed_workspace_bytes(int64_t m, int64_t k, int64_t n,
                                      int32_t channels,
                                      const rnsmx_plan_t *plan);

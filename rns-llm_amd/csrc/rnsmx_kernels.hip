@@ -1915,9 +1915,13 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   g.mods = *mods;
   GemmChoice c{};
   if (int32_t rc = packed ? packed_plan_from(plan, g, c, a_dtype) : plan_from(plan, g, araw, true, c, true)) return rc;
-  if (c.kind == kUnits && (plan == nullptr || plan->kind == kAuto) &&
-      workspace_bytes < prepared_layout(araw, m, k, R, xchg_bytes(c, g)).total)
-    c = auto_plan(g, araw, true);  // a workspace made for more rows may hold no exchange area
+  // a workspace made for more rows may hold no exchange area
+  if (plan == nullptr || plan->kind == kAuto) {
+    if (c.kind == kUnits && workspace_bytes < prepared_layout(araw, m, k, R, xchg_bytes(c, g)).total)
+      c = auto_plan(g, araw, true);
+    else if (c.kind == kBytesLds && workspace_bytes < packed_layout(m, kp, R, xchg_bytes(c, g)).total)
+      c.splits = 1;
+  }
   const bool bytes = c.kind == kBytesRows || c.kind == kBytesLds;
   const PreparedLayout l = packed ? packed_layout(m, kp, R, xchg_bytes(c, g))
                                   : prepared_layout(araw, m, k, R, xchg_bytes(c, g));

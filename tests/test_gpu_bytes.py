@@ -2,6 +2,7 @@
 kernel over fragments, waves and ragged rows, the tiles over ragged edges, K
 steps that fill no trip and K splits, float outputs, and sets too small for
 the product, against the exact product taken to the set's centered range."""
+import ctypes
 from math import prod
 
 import numpy as np
@@ -9,6 +10,7 @@ import pytest
 import torch
 
 from oracle import rns_oracle as ro
+from rns_llm_amd import _native
 
 pytestmark = pytest.mark.gpu
 
@@ -130,6 +132,26 @@ def test_replays_of_a_captured_split(backend):
         torch.cuda.synchronize()
         assert torch.equal(ws.output.cpu(), want)
         assert torch.equal(backend.matmul_prepared_fused(x, prepared, workspace=ws, plan=plan).cpu(), want)
+
+
+@pytest.mark.parametrize("m", [70, 130])
+@pytest.mark.parametrize("dtype", [torch.int8, torch.int16])
+def test_split_without_an_exchange_area(backend, m, dtype):
+    """A workspace with room for the planes alone: the same product, unsplit."""
+    k, n = 4096, 200
+    a, w, want = operands(m, k, n, dtype, m)
+    prepared = backend.prepare_weight_packed_nk(w.cuda(), DENSE6)
+    lib, mods = _native.lib(), _native.make_moduli(DENSE6)
+    whole = _native.Plan(10, 4, 1, 0, 1, 0)
+    small = lib.rnsmx_packed_workspace_bytes(m, k, n, 6, ctypes.byref(whole))
+    assert small < lib.rnsmx_packed_workspace_bytes(m, k, n, 6, None)
+    x = a.cuda()
+    workspace = torch.zeros((small,), dtype=torch.uint8, device="cuda")
+    out = torch.empty((m, n), dtype=torch.int64, device="cuda")
+    _native.check(lib.rnsmx_matmul_packed_fused(
+        x.data_ptr(), _native.dtype_code(dtype), m, k, n, prepared.packed.data_ptr(), ctypes.byref(mods), None, 0, None,
+        None, None, workspace.data_ptr(), small, out.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out.cpu(), want)
 
 
 def test_plans_refused(backend):

@@ -1,5 +1,9 @@
-"""Sizes at which a kernel's addressing ends: the host refuses its plan."""
+"""Sizes at which a kernel's addressing ends: the host refuses its plan.  And
+workspaces made for other calls: the host takes a plan that fits them."""
 import ctypes
+
+import pytest
+import torch
 
 from rns_llm_amd import _native
 
@@ -18,3 +22,30 @@ def test_byte_product_planes_stay_below_32_bit_offsets():
             assert lib.rnsmx_packed_workspace_bytes(most + 1, k, 64, 6, ctypes.byref(plan)) == -1
         # an automatic plan still serves them, by residue channels
         assert lib.rnsmx_packed_workspace_bytes(most + 1, k, 64, 6, None) > 0
+
+
+def runs_in(lib, mods, dtype, m, k, n, nbytes):
+    """Whether a packed product accepts a workspace of nbytes.  Without a GPU a
+    call that passes its checks ends at the launch, which reads nothing."""
+    fake = 1 << 20
+    return lib.rnsmx_matmul_packed_fused(fake, dtype, m, k, n, fake, ctypes.byref(mods), None, 0, None, None, None,
+                                         fake, nbytes, fake, None) != _native.ESPACE
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="calls that pass the checks would launch on made-up pointers")
+@pytest.mark.parametrize("k,n", [(2048, 64), (2048, 333), (4096, 4096), (4096, 12288), (8192, 768)])
+@pytest.mark.parametrize("moduli", [(255, 253, 251), (255, 253, 251, 247, 241, 239)], ids=len)
+def test_a_packed_workspace_serves_fewer_rows(moduli, k, n):
+    """The room that residue channels of `most` rows take serves every call of
+    up to `most` rows: a byte product whose K split needs more runs unsplit."""
+    lib = _native.lib()
+    mods = _native.make_moduli(moduli)
+    for most in (24, 48, 64, 128, 256, 512, 1024):
+        # the planes and row terms of residue channels, the counters and the row norms
+        up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+        planes = up(2 * len(moduli) * most * k + 4 * len(moduli) * ((most + 63) // 64 * 64 + 64))
+        room = _native.SPLIT_TICKETS * 4 + max(planes, up(16 * k * 16 if most <= 32 else 0)) + up(8 * (most + 1))
+        for m in (1, 9, 17, 24, 33, 48, 64, 65, 128, 200, 256, 512, 1024):
+            if m <= most:
+                for dtype in (_native.INT8, _native.INT16):
+                    assert runs_in(lib, mods, dtype, m, k, n, room), (most, m, dtype)
