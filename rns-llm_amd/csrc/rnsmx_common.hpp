@@ -22,6 +22,13 @@ inline int32_t fail(int32_t code, const char *what) {
 
 inline int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
+// Whether [a, a + an) and [b, b + bn) share a byte: a kernel that writes one
+// while its other workgroups still read the other needs them apart.
+inline bool ranges_meet(const void *a, int64_t an, const void *b, int64_t bn) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + static_cast<uintptr_t>(bn) && y < x + static_cast<uintptr_t>(an);
+}
+
 // Largest |centered residue| of the set: floor(max(m) / 2).
 inline int32_t max_half(const rnsmx_moduli_t &mods) {
   int32_t h = 0;

@@ -2499,9 +2499,13 @@ int32_t rnsmx_linear_forward(const void *x_dev, int32_t x_dtype, int32_t rows, i
               static_cast<long long>(l.total));
     return RNSMX_ESPACE;
   }
+  // A few rows: quantized inside the product, one launch, whose workgroups read
+  // all of x: outputs written over the activations take the quantizer's own
+  // kernels, which have read x before the product starts.
+  const int64_t size = x_dtype == RNSMX_FLOAT32 ? 4 : 2;
   if (linear_rows_fits(rows, k, n, *mods, quant_bits, adaptive != nullptr && adaptive->min_channels != 0,
-                       aligned16(x_dev))) {
-    // a few rows: quantized inside the product, one launch
+                       aligned16(x_dev)) &&
+      !ranges_meet(x_dev, size * rows * k, out_dev, size * rows * n)) {
     if (!x_dev || !packed_dev || !out_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
     GemmArgs g = plan_args(rows, n, k, mods->channels, true);
     g.mods = *mods;

@@ -69,3 +69,21 @@ def test_zero_input_and_replays(backend):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, layer(x))
+
+
+@pytest.mark.parametrize("shift", [0, -256, 512])
+@pytest.mark.parametrize("rows,k,n", [(1, 768, 768), (4, 1024, 1024), (3, 512, 1000)])
+def test_outputs_over_the_activations(backend, rows, k, n, shift):
+    """The library call with out_dev inside x_dev: as into another buffer."""
+    layer = layer_of(backend, k, n, torch.float16)
+    x = torch.randn((rows, k), generator=torch.Generator().manual_seed(n)).to(device="cuda", dtype=torch.float16)
+    with torch.no_grad():
+        want = layer(x)
+        call = layer._bind_linear()
+        buffer = torch.zeros((rows * max(k, n) + 2048,), dtype=torch.float16, device="cuda")
+        scratch = backend.create_linear_scratch(call, rows, x.device)
+        for _ in range(5):
+            inside = buffer[1024:1024 + rows * k].view(rows, k).copy_(x)
+            out = buffer[1024 + shift:1024 + shift + rows * n].view(rows, n)
+            call(inside, rows, out, scratch)
+            assert torch.equal(out, want)
