@@ -1958,11 +1958,13 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   const bool rows = packed && c.kind == kRows;
   const int ab = a_dtype == RNSMX_INT8 ? 1 : 2;  // bytes per activation (byte products)
   if (c.kind == kBytesRows) {
-    // rows read as they are; rows that are not 16-byte aligned are copied
-    // to padded ones first
+    // rows read as they are; rows that are not 16-byte aligned, or that the
+    // outputs are written over, are copied to padded ones first
     g.a = static_cast<const int8_t *>(a_dev);
     g.a_ld = g.a_k = k;
-    if (static_cast<int64_t>(k) * ab % 16 != 0) {
+    const int64_t out_size = out_dtype == RNSMX_INT64 ? 8 : out_dtype == RNSMX_FLOAT32 ? 4 : 2;
+    if (static_cast<int64_t>(k) * ab % 16 != 0 ||
+        ranges_meet(a_dev, static_cast<int64_t>(m) * k * ab, out_dev, out_size * m * n)) {
       if (int32_t rc = launch_pad_rows(g.a, m, static_cast<int64_t>(k) * ab, kp * ab, a_res, st)) return rc;
       g.a = a_res;
       g.a_ld = kp;

@@ -154,6 +154,27 @@ def test_split_without_an_exchange_area(backend, m, dtype):
     assert torch.equal(out.cpu(), want)
 
 
+@pytest.mark.parametrize("m", [1, 8, 20, 70])
+def test_outputs_over_the_activations(backend, m):
+    """Float outputs written where the int16 activations lie, and int64 ones
+    that begin inside them: as into another buffer."""
+    k = n = 512
+    a, w, want = operands(m, k, n, torch.int16, m)
+    prepared = backend.prepare_weight_packed_nk(w.cuda(), DENSE6)
+    scales = dict(a_scale=torch.tensor([3e-5], device="cuda"), w_scale=torch.full((n,), 1e-4, device="cuda"))
+    out = torch.empty((m, n), dtype=torch.float16, device="cuda")
+    backend.matmul_prepared_fused(a.cuda(), prepared, out=out, **scales)
+    buffer = torch.empty((5 * m * k,), dtype=torch.int16, device="cuda")
+    for _ in range(5):
+        x = buffer[:m * k].view(m, k).copy_(a)
+        got = backend.matmul_prepared_fused(x, prepared, out=x.view(torch.float16), **scales)
+        assert torch.equal(got, out)
+        x.copy_(a)
+        ws = backend.create_workspace(device=x.device, channels=6, m=m, n=n, k=k)
+        ws.output = buffer[m * k - 64:m * k - 64 + 4 * m * n].view(torch.int64).view(m, n)
+        assert torch.equal(backend.matmul_prepared_fused(x, prepared, workspace=ws).cpu(), want)
+
+
 def test_plans_refused(backend):
     a, w, _ = operands(20, 64, 16, torch.int32, 1)
     prepared = backend.prepare_weight_packed_nk(w.cuda(), DENSE6)
