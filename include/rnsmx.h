@@ -244,8 +244,10 @@ int32_t rnsmx_matmul_prepared_fused(
  * rows one after the other -> out_dev [sum rows][N] int64, as
  * rnsmx_matmul_prepared_fused (rnsmx_matmul_packed_fused) of their
  * concatenation, which staging_dev ([sum rows][K], 16-byte aligned) holds
- * afterwards.  Workspace as for that call.  One launch for up to 16 int8 rows
- * (4 channels, K a multiple of 16, 16-byte aligned requests).
+ * afterwards.  No request may overlap staging_dev (RNSMX_EINVAL): rows are
+ * copied there while others are still read.  Workspace as for that call.  One
+ * launch for up to 16 int8 rows (4 channels, K a multiple of 16, 16-byte
+ * aligned requests clear of out_dev).
  * Replaces the concatenation and product of matmul_prepared_fused_requests
  * (cuda_backend.py:647-703).
  */

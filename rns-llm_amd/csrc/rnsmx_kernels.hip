@@ -2081,16 +2081,24 @@ int32_t rnsmx_matmul_requests(const void *const *requests, const int32_t *rows, 
     return fail(RNSMX_EINVAL, "bad request batch");
   if (!staging_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
   int64_t m = 0;
-  bool aligned = aligned16(staging_dev);
   for (int32_t i = 0; i < count; ++i) {
     if (rows[i] < 1 || !requests[i]) return fail(RNSMX_EINVAL, "every request needs a row");
     m += rows[i];
-    aligned = aligned && aligned16(requests[i]);
   }
   if (m > INT32_MAX) return fail(RNSMX_EINVAL, "bad request batch");
+  const int64_t row_bytes = static_cast<int64_t>(k) * static_cast<int64_t>(dtype_size(a_dtype));
+  // whether the one-launch kernel can read every request in place: aligned, and
+  // clear of the outputs it stores meanwhile (a gather reads them first)
+  bool in_place = aligned16(staging_dev);
+  for (int32_t i = 0; i < count; ++i) {
+    if (ranges_meet(requests[i], rows[i] * row_bytes, staging_dev, m * row_bytes))
+      return fail(RNSMX_EINVAL, "a request overlaps the staging buffer");
+    in_place = in_place && aligned16(requests[i]) &&
+               !ranges_meet(requests[i], rows[i] * row_bytes, out_dev, 8 * m * n);
+  }
   hipStream_t st = static_cast<hipStream_t>(stream);
   int8_t *staging = static_cast<int8_t *>(staging_dev);
-  if (packed_form == 0 && aligned && n > 0 && request_rows_fits(m, k, *mods, a_dtype)) {
+  if (packed_form == 0 && in_place && n > 0 && request_rows_fits(m, k, *mods, a_dtype)) {
     if (!packed_dev || !out_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
     GemmArgs g = plan_args(m, n, k, mods->channels, true);
     g.mods = *mods;
@@ -2108,7 +2116,6 @@ int32_t rnsmx_matmul_requests(const void *const *requests, const int32_t *rows, 
     launch_request_rows(g, row, staging, st);
     return check_launch("request_rows");
   }
-  const int64_t row_bytes = static_cast<int64_t>(k) * static_cast<int64_t>(dtype_size(a_dtype));
   int64_t at = 0;
   for (int32_t i0 = 0; i0 < count; i0 += kGatherMost) {
     GatherArgs a{};

@@ -69,3 +69,26 @@ def test_requests_inside_the_staging_buffer_are_refused(backend, rows):
     half = rows[0]
     with pytest.raises(RuntimeError):
         backend.matmul_prepared_fused_requests([ws.activations[half:], ws.activations[:half]], prepared, workspace=ws)
+
+
+@pytest.mark.parametrize("rows", [(1, 1), (4, 12), (20, 20)])
+def test_outputs_over_a_request(backend, rows):
+    """Outputs written where a request lies, or begin inside it."""
+    k, n = 512, 64
+    gen = torch.Generator().manual_seed(sum(rows))
+    w = torch.randint(-127, 128, (n, k), generator=gen, dtype=torch.int32).to(torch.int8)
+    prepared = backend.prepare_weight_nk(w.cuda(), DENSE4)
+    ws = backend.create_request_batch_workspace(device=torch.device("cuda"), dtype=torch.int8, rows_per_request=rows, k=k,
+                                                channels=4, n=n)
+    m, given = sum(rows), [torch.randint(-128, 128, (r, k), generator=gen, dtype=torch.int32).to(torch.int8) for r in rows]
+    buffer = torch.empty((2 * m * (k + 8 * n),), dtype=torch.int8, device="cuda")
+    for lo in (0, k // 2):
+        ws.fused.output = buffer[lo:lo + 8 * m * n].view(torch.int64).view(m, n)
+        for _ in range(5):
+            requests, at = [], 0
+            for r, x in zip(rows, given):
+                requests.append(buffer[at:at + r * k].view(r, k).copy_(x))
+                at += r * k
+            outs = backend.matmul_prepared_fused_requests(requests, prepared, workspace=ws)
+            for x, out in zip(given, outs):
+                assert torch.equal(out.cpu(), exact(x, w))

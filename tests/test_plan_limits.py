@@ -49,3 +49,19 @@ def test_a_packed_workspace_serves_fewer_rows(moduli, k, n):
             if m <= most:
                 for dtype in (_native.INT8, _native.INT16):
                     assert runs_in(lib, mods, dtype, m, k, n, room), (most, m, dtype)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="calls that pass the checks would launch on made-up pointers")
+def test_requests_stay_clear_of_the_staging_buffer():
+    lib, mods = _native.lib(), _native.make_moduli((255, 253, 251, 247))
+    staging, k, rows = 1 << 20, 64, (3, 2)
+
+    def code(*at):
+        return lib.rnsmx_matmul_requests((ctypes.c_void_p * 2)(*at), (ctypes.c_int32 * 2)(*rows), 2, _native.INT8, k, 16,
+                                         1 << 22, ctypes.byref(mods), 0, staging, 1 << 23, 1 << 30, 1 << 24, None)
+
+    end = staging + 5 * k
+    for at in ((staging, end), (end, staging), (end - 1, end + 512), (end, staging - 2 * k + 1)):
+        assert code(*at) == _native.EINVAL and b"staging" in lib.rnsmx_last_error()
+    for at in ((end, end + 3 * k), (staging - 3 * k, end), (end + 16, staging - 2 * k)):
+        assert code(*at) == _native.ELAUNCH  # no device: every check passed
