@@ -261,11 +261,12 @@ int32_t rnsmx_matmul_requests(const void *const *requests, const int32_t *rows,
 
 /*
  * Both operands plain integers, used once: a_dev [M][K] and b_dev [K][N], both
- * int8, int16 or int32 (row-major) -> exact out_dev [M][N] int64.  Encodes B
- * straight into the fragment-major order of rnsmx_prepare_weight in the
- * workspace and runs the prepared-weight product; the workspace may hold
- * anything before the call (rnsmx_wide_workspace_bytes) and its counters are
- * zero after it.
+ * int8, int16 or int32 (row-major; a_dev 16-byte aligned) -> exact out_dev
+ * [M][N] int64.  Encodes B straight into the fragment-major order of
+ * rnsmx_prepare_weight in the workspace and runs the prepared-weight product;
+ * the workspace may hold anything before the call (rnsmx_wide_workspace_bytes)
+ * and its counters are zero after it.  RNSMX_EINVAL where an operand overlaps
+ * the workspace, or out_dev an int8 A of K a multiple of 16 (read in place).
  * Replaces the chain encode_centered (both operands) -> matmul_centered_fused
  * of CudaRNSBackend.matmul_wide (cuda_backend.py:733-799).
  */

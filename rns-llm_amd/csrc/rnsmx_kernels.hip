@@ -2172,9 +2172,14 @@ int32_t rnsmx_matmul_wide(const void *a_dev, const void *b_dev, int32_t dtype, i
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t at = wide_weight_at(m, k, n, mods->channels);
   int8_t *ws = static_cast<int8_t *>(workspace_dev);
+  const int64_t size = static_cast<int64_t>(dtype_size(dtype)), a_bytes = size * m * k;
+  if (ranges_meet(a_dev, a_bytes, workspace_dev, need) || ranges_meet(b_dev, size * k * n, workspace_dev, need))
+    return fail(RNSMX_EINVAL, "an operand overlaps the workspace");
   // the counters of the split that the product will take are cleared by the
   // encoder, so the workspace may hold anything before the call
   const bool araw = raw_route(dtype, k, *mods, nullptr);
+  if (araw && k % 16 == 0 && ranges_meet(a_dev, a_bytes, out_dev, int64_t{8} * m * n))
+    return fail(RNSMX_EINVAL, "the outputs overlap int8 activations that are read in place");
   const GemmArgs g = plan_args(m, n, k, mods->channels, araw);
   GemmChoice c{};
   if (int32_t rc = plan_from(nullptr, g, araw, true, c, true)) return rc;

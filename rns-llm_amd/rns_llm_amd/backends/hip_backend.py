@@ -224,6 +224,12 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _overlap(t: torch.Tensor, u: torch.Tensor) -> bool:
+    """Whether two contiguous tensors share a byte."""
+    lo, hi = t.data_ptr(), u.data_ptr()
+    return lo < hi + u.nbytes and hi < lo + t.nbytes
+
+
 class LinearCall:
     """``RNSLinear.forward``'s device work bound to one prepared weight: one
     ``rnsmx_linear_forward`` call per forward (activation quantization, then
@@ -1108,7 +1114,9 @@ class HipRNSBackend:
                 workspace = self.create_workspace(device=a.device, channels=len(mods), m=m, n=n)
             self._check_workspace(workspace, channels=len(mods), m=m, n=n, device=a.device)
             scratch = self._scratch(workspace, self._wide_bytes(m, k, n, len(mods)))
-            return self._wide_call(a, b, mods, scratch, workspace.output)
+            if not (_overlap(a, workspace.output) or _overlap(a, scratch) or _overlap(b, scratch)):
+                return self._wide_call(a, b, mods, scratch, workspace.output)
+            # operands inside the workspace: the chain encodes both first
         a_res, b_res, mods = self._encode_operands(a, b, moduli)
         return self.matmul_centered_fused(a_res, b_res, mods, lut_channels=lut_channels, workspace=workspace)
 

@@ -96,3 +96,24 @@ def test_unprepared_refusals(backend):
             bad()
     # an empty batch
     assert backend.matmul_wide(a[:0], b, DENSE4).shape == (0, 8)
+
+
+@pytest.mark.parametrize("dtype", [torch.int8, torch.int16])
+@pytest.mark.parametrize("where", ["output", "accumulators"])
+@pytest.mark.parametrize("operand", ["a", "b"])
+def test_operands_inside_the_workspace(backend, operand, where, dtype):
+    """An operand that lies where the outputs or the scratch will be."""
+    m, k, n = 64, 128, 96
+    a, b = ints((m, k), 126, dtype, 3), ints((k, n), 126, dtype, 4)
+    ws = backend.create_workspace(device=torch.device("cuda"), channels=6, m=m, n=n)
+    want = exact(a, b)
+    # grown to this shape's size, so that the next call keeps the buffer
+    assert torch.equal(backend.matmul_wide_fused(a.cuda(), b.cuda(), DENSE6, workspace=ws).cpu(), want)
+    x, y = a.cuda(), b.cuda()
+    for _ in range(5):
+        at = getattr(ws, where).view(-1).view(torch.int8)
+        at = at[at.numel() // 2 // 16 * 16:] if where == "accumulators" else at
+        inside = at[:(x if operand == "a" else y).nbytes].view(dtype).view((x if operand == "a" else y).shape)
+        pair = (inside.copy_(x), y) if operand == "a" else (x, inside.copy_(y))
+        assert torch.equal(backend.matmul_wide_fused(*pair, DENSE6, workspace=ws).cpu(), want)
+        ws.accumulators.zero_()  # its counters were written over

@@ -65,3 +65,24 @@ def test_requests_stay_clear_of_the_staging_buffer():
         assert code(*at) == _native.EINVAL and b"staging" in lib.rnsmx_last_error()
     for at in ((end, end + 3 * k), (staging - 3 * k, end), (end + 16, staging - 2 * k)):
         assert code(*at) == _native.ELAUNCH  # no device: every check passed
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="calls that pass the checks would launch on made-up pointers")
+@pytest.mark.parametrize("dtype,size", [(_native.INT8, 1), (_native.INT16, 2)])
+def test_unprepared_operands_stay_clear_of_what_is_written(dtype, size):
+    lib, mods = _native.lib(), _native.make_moduli((255, 253, 251, 247))
+    m, k, n, ws = 32, 64, 48, 1 << 24
+    need = lib.rnsmx_wide_workspace_bytes(m, k, n, 4)
+
+    def code(a=1 << 20, b=1 << 21, out=1 << 22, width=k):
+        return lib.rnsmx_matmul_wide(a, b, dtype, m, width, n, ctypes.byref(mods), ws, need, out, None)
+
+    assert code() == _native.ELAUNCH  # no device: every check passed
+    for bad in (dict(a=ws), dict(b=ws + need - 16), dict(a=ws + 16 - size * m * k), dict(b=ws + 1 - size * k * n)):
+        assert code(**bad) == _native.EINVAL and b"workspace" in lib.rnsmx_last_error()
+    assert code(b=ws - size * k * n) == _native.ELAUNCH and code(a=ws + (need + 15) // 16 * 16) == _native.ELAUNCH
+    # int8 rows are read in place where K is a multiple of 16; others are copied first
+    over = (1 << 22) + 16
+    assert code(a=over) == (_native.EINVAL if size == 1 else _native.ELAUNCH)
+    assert code(a=over, width=k - 1) == _native.ELAUNCH
+    assert code(b=over) == _native.ELAUNCH
