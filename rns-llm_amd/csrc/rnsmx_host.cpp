@@ -53,6 +53,9 @@ static FracSet make_frac_set(const rnsmx_moduli_t &mods) {
   FracSet s{};
   const int channels = mods.channels;
   if (channels < 1 || channels > 6) return s;
+  // a set that rnsmx_moduli_init has not filled: no constants, and no division by zero
+  for (int c = 0; c < channels; ++c)
+    if (mods.moduli[c] < 2) return s;
   for (int p = 1; p <= channels; ++p) {
     for (int c = 0; c < p; ++c) {
       const int m = mods.moduli[c];

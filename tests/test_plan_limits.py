@@ -1,6 +1,10 @@
-"""Sizes at which a kernel's addressing ends: the host refuses its plan.  And
-workspaces made for other calls: the host takes a plan that fits them."""
+"""Sizes at which a kernel's addressing ends: the host refuses its plan.
+Workspaces made for other calls: the host takes a plan that fits them.  And
+arguments that a C caller can get wrong: an error code, not the process."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -86,3 +90,26 @@ def test_unprepared_operands_stay_clear_of_what_is_written(dtype, size):
     assert code(a=over) == (_native.EINVAL if size == 1 else _native.ELAUNCH)
     assert code(a=over, width=k - 1) == _native.ELAUNCH
     assert code(b=over) == _native.ELAUNCH
+
+
+UNFILLED = """
+import ctypes, sys
+from rns_llm_amd import _native
+lib, fake = _native.lib(), 1 << 20
+for values in ((0, 0), (0, 251), (251, 0, 1), (1, 1), (-3, 5), (4, 2, 0, 0, 0, 0)):
+    print(values, flush=True)
+    mods = _native.Moduli(channels=len(values))
+    mods.moduli[:len(values)] = values
+    lib.rnsmx_matmul_prepared_fused(fake, _native.INT8, 4, 64, 16, fake, ctypes.byref(mods), None, 0, None, None, None,
+                                    fake, 1 << 30, fake, None)
+"""
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="calls that pass the checks would launch on made-up pointers")
+def test_a_set_that_was_never_initialised_ends_no_process():
+    """A moduli block whose channels are set but whose constants are not: an
+    error code (the launch's, without a GPU), and the process goes on."""
+    path = os.pathsep.join(p for p in sys.path if p)
+    done = subprocess.run([sys.executable, "-c", UNFILLED], env=dict(os.environ, PYTHONPATH=path), capture_output=True,
+                          text=True, timeout=120)
+    assert done.returncode == 0, done.stdout + done.stderr
