@@ -969,6 +969,7 @@ class HipRNSBackend:
         ``clone_outputs``)."""
         if len(requests) == 0:
             raise ValueError("no requests to batch")
+        requests = tuple(requests)  # any sized container
         for index, request in enumerate(requests):
             if not (request.is_cuda and request.ndim == 2 and request.is_contiguous()):
                 self._validate_matrix(request, f"request {index}", 2)
@@ -990,7 +991,7 @@ class HipRNSBackend:
                              f"requests are {rows} x K={k}")
         merged = self._merged_product(requests, rows, prepared_weight, lut_channels, workspace)
         if merged is None:
-            torch.cat(tuple(requests), dim=0, out=workspace.activations)
+            torch.cat(requests, dim=0, out=workspace.activations)
             merged = self.matmul_prepared_fused(workspace.activations, prepared_weight,
                                                 lut_channels=lut_channels, workspace=workspace.fused)
         views = merged.split(rows)

@@ -1,0 +1,30 @@
+"""Arguments of the Python entry points, checked before anything reaches the
+GPU: stand-ins with a tensor's attributes take the place of device tensors."""
+from collections import deque
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from rns_llm_amd import HipRNSBackend
+
+
+def matrix(rows, cols, dtype=torch.int8):
+    return SimpleNamespace(is_cuda=True, ndim=2, is_contiguous=lambda: True, dtype=dtype, device="cuda:0",
+                           shape=(rows, cols), numel=lambda: rows * cols)
+
+
+def backend():
+    return object.__new__(HipRNSBackend)  # no GPU here
+
+
+@pytest.mark.parametrize("held", [list, tuple, deque, lambda r: dict(enumerate(r)).values()],
+                         ids=["list", "tuple", "deque", "values"])
+def test_requests_in_any_sized_container(held):
+    """Anything with a length that can be iterated: the checks go on to what
+    is wrong with the requests themselves."""
+    prepared = SimpleNamespace(k=64)
+    with pytest.raises(ValueError, match="widths"):
+        backend().matmul_prepared_fused_requests(held([matrix(1, 64), matrix(2, 32)]), prepared)
+    with pytest.raises(ValueError, match="dtypes"):
+        backend().matmul_prepared_fused_requests(held([matrix(1, 64), matrix(2, 64, torch.int16)]), prepared)
