@@ -1010,7 +1010,7 @@ class HipRNSBackend:
         if (dtype != requests[0].dtype or dtype not in _DTYPE_MAX_ABS or device != requests[0].device
                 or device != prepared.packed.device or tuple(staging.shape) != (m, prepared.k)
                 or not staging.is_contiguous() or staging.data_ptr() % 16 or lut_channels not in (0, 1, 2)
-                or lut_channels > channels or n == 0):
+                or lut_channels > channels or n == 0 or 0 in rows):
             return None
         pointers = [r.data_ptr() for r in requests]
         begin = staging.data_ptr()

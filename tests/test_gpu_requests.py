@@ -92,3 +92,19 @@ def test_outputs_over_a_request(backend, rows):
             outs = backend.matmul_prepared_fused_requests(requests, prepared, workspace=ws)
             for x, out in zip(given, outs):
                 assert torch.equal(out.cpu(), exact(x, w))
+
+
+def test_a_request_without_rows(backend):
+    """A batch workspace put together by hand may hold a request of no rows."""
+    from rns_llm_amd.backends.hip_backend import RNSRequestBatchWorkspace
+
+    gen = torch.Generator().manual_seed(2)
+    w, x = (torch.randint(-127, 128, shape, generator=gen, dtype=torch.int32).to(torch.int8) for shape in ((16, 64), (3, 64)))
+    prepared, dev = backend.prepare_weight_nk(w.cuda(), DENSE4), torch.device("cuda")
+    ws = RNSRequestBatchWorkspace(activations=torch.empty((3, 64), dtype=torch.int8, device=dev),
+                                  fused=backend.create_workspace(device=dev, channels=4, m=3, n=16, k=64),
+                                  rows_per_request=(1, 0, 2), k=64)
+    rows = x.cuda()
+    outs = backend.matmul_prepared_fused_requests([rows[:1], rows[1:1], rows[1:]], prepared, workspace=ws)
+    assert [o.shape[0] for o in outs] == [1, 0, 2]
+    assert torch.equal(torch.cat(outs).cpu(), exact(x, w))
