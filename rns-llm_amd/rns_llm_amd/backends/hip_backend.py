@@ -1060,7 +1060,7 @@ class HipRNSBackend:
                 and a.dtype == b.dtype and a.dtype in _DTYPE_MAX_ABS and a.device == b.device
                 and a.shape[1] == b.shape[0] and a.numel() and b.numel()):
             return None
-        mods = tuple(moduli)
+        mods = tuple(map(int, moduli))  # plain integers: they key the device constants
         if not self.mfma_compatible(k=int(a.shape[1]), n=int(b.shape[1]), moduli=mods, device=a.device):
             return None
         return mods

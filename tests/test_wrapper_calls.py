@@ -28,3 +28,12 @@ def test_requests_in_any_sized_container(held):
         backend().matmul_prepared_fused_requests(held([matrix(1, 64), matrix(2, 32)]), prepared)
     with pytest.raises(ValueError, match="dtypes"):
         backend().matmul_prepared_fused_requests(held([matrix(1, 64), matrix(2, 64, torch.int16)]), prepared)
+
+
+@pytest.mark.parametrize("moduli", [torch.tensor([255, 253, 251]), ["255", "253", "251"], (255.0, 253.0, 251.0),
+                                    iter((255, 253, 251))], ids=["tensor", "text", "float", "iterator"])
+def test_unprepared_moduli_become_integers(moduli):
+    """The set keys the cache of device constants: a fresh tensor's elements
+    would be a new entry on every call."""
+    mods = backend()._wide_operands(matrix(4, 64), matrix(64, 8), moduli)
+    assert mods == (255, 253, 251) and all(type(m) is int for m in mods)
