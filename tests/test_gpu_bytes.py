@@ -62,6 +62,24 @@ def test_tiles(backend, m, k, n, mb, dtype):
     assert torch.equal(run(backend, a, w, DENSE6, (10, mb, 1, 0)), want)
 
 
+# the longest K whose int32 sums hold: every middle product of the weight's and
+# the activations' bytes is 2^14, twice per K index, 2145386496 of 2^31 - 1
+@pytest.mark.parametrize("plan", [None, (9, 4, 1, 1), (9, 4, 1, 4), (10, 4, 1, 0), (10, 8, 1, 0), (10, 8, 1, 0, 4)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.int8, torch.int16])
+def test_longest_k(backend, plan, dtype):
+    lim = 128 if dtype == torch.int8 else 32768
+    for k in (65472, 65471, 65473):
+        a, w = (torch.empty((3, k), dtype=t) for t in (dtype, torch.int16))
+        for x, top in ((a, lim), (w, 32768)):
+            x[0], x[1], x[2] = -top, top - 1, torch.arange(k) % (2 * top) - top
+        want = torch.from_numpy(ro.exact_matmul(a.numpy(), w.t().numpy()))
+        if k == 65473 and plan is not None:
+            with pytest.raises(ValueError, match="65472"):
+                run(backend, a, w, DENSE6, plan)
+        else:
+            assert torch.equal(run(backend, a, w, DENSE6, plan), want)
+
+
 @pytest.mark.parametrize("splits,tail", [(2, 0), (3, 0), (8, 0), (2, 1)])
 @pytest.mark.parametrize("mb", [4, 8])
 @pytest.mark.parametrize("dtype", [torch.int8, torch.int16])

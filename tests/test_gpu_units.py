@@ -7,6 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from oracle import rns_oracle as ro
 from rns_llm_amd import HipRNSBackend
 
 pytestmark = pytest.mark.gpu
@@ -63,17 +64,28 @@ def test_channel_units_float_outputs(m, n, out_dtype, plan):
     assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("most", [3, 200, 32767])
+@pytest.mark.parametrize("plan", [None, SMALL, LARGE])
 @pytest.mark.parametrize("m, n, k", [(96, 640, 1024), (200, 515, 513)])
-def test_channel_units_adaptive_prefix(m, n, k, most):
-    """Units past the prefix the activations need end at once."""
-    gen = torch.Generator().manual_seed(most)
-    a = torch.randint(-most, most + 1, (m, k), generator=gen)
+def test_channel_units_adaptive_prefix(m, n, k, plan):
+    """Units past the prefix the activations need end at once.  Prefixes of
+    different lengths alternate on one workspace, so a ticket that one call
+    left would end the next one early."""
+    gen = torch.Generator().manual_seed(k)
     w = torch.randint(-32767, 32768, (n, k), generator=gen)
+    w[0, 0] = 32767
     backend = HipRNSBackend()
     prepared = backend.prepare_weight_adaptive_nk(w.to(torch.int16).cuda(), MODULI, min_channels=2)
-    out, meta = backend.matmul_prepared_adaptive_fused(a.to(torch.int16).cuda(), prepared, return_metadata=True)
-    assert torch.equal(out.cpu(), (a.double() @ w.double().t()).to(torch.int64))
+    workspaces = {6: backend.create_workspace(device=torch.device("cuda"), channels=6, m=m, n=n, k=k)}
+    seen = []
+    for most in (1, 32767, 2000, 1, 2000, 32767):
+        a = torch.randint(-most, most + 1, (m, k), generator=gen)
+        out, meta = backend.matmul_prepared_adaptive_fused(a.to(torch.int16).cuda(), prepared, return_metadata=True,
+                                                           workspace_by_channels=workspaces, plan=plan)
+        channels, bound, capacity = ro.adaptive_select(a.numpy(), 32767, MODULI, min_channels=2)
+        assert dict(meta) == {"channels": channels, "bound": bound, "capacity": capacity}
+        assert torch.equal(out.cpu(), (a.double() @ w.double().t()).to(torch.int64))
+        seen.append(channels)
+    assert seen[:3] == ([4, 6, 5] if k == 1024 else [4, 5, 5])
 
 
 def test_channel_units_replayed():

@@ -28,6 +28,48 @@ def test_byte_product_planes_stay_below_32_bit_offsets():
         assert lib.rnsmx_packed_workspace_bytes(most + 1, k, 64, 6, None) > 0
 
 
+def room(query, m, n, k, channels, plan=None):
+    return query(m, k, n, channels, None if plan is None else ctypes.byref(_native.Plan(*plan)))
+
+
+# (M, N, K, channels) on both sides of where an automatic plan takes channel
+# units (kind 11), and their two tiles; None: the plan without them
+@pytest.mark.parametrize("shape,units", [
+    ((16, 4096, 4096, 6), None), ((17, 4096, 4096, 6), (11, 2, 1, 0)),           # rows
+    ((17, 768, 768, 6), None),                                                   # short K: the stream kernel
+    ((64, 2304, 768, 5), (11, 2, 1, 0)), ((160, 1536, 1024, 6), (11, 2, 1, 0)),
+    ((200, 515, 513, 6), (11, 2, 1, 0)), ((40, 12288, 4096, 6), (11, 4, 2, 0)),
+    ((512, 768, 768, 6), None), ((300, 514, 576, 6), None), ((512, 12288, 4096, 6), None),
+    ((512, 2048, 5120, 6), None),                                                # past four workgroups per CU
+], ids=str)
+def test_where_channel_units_are_taken(shape, units):
+    """Read from the room the automatic plan asks for: the units' exchange of a
+    byte per channel and element, or that of the plan rnsmx_gemm_plan gives."""
+    lib = _native.lib()
+    query, (m, n, k, channels) = lib.rnsmx_prepared_workspace_bytes, shape
+    other = _native.Plan()
+    _native.check(lib.rnsmx_gemm_plan(m, n, k, channels, 0, ctypes.byref(other)))
+    rooms = {plan: room(query, *shape, plan=plan) for plan in ((11, 2, 1, 0), (11, 4, 2, 0), other.as_tuple())}
+    taken = rooms.pop(units or other.as_tuple())
+    assert room(query, *shape) == taken and taken not in rooms.values()  # so the room tells which
+
+
+# N = 12288: 128 tiles of 64 x 96; K of no whole 256, so that int32 activations
+# (the channel form) never split
+@pytest.mark.parametrize("shape,splits", [
+    ((17, 12288, 4160), 2), ((64, 12288, 4160), 2), ((65, 12288, 4160), 1), ((64, 12384, 4160), 1),
+    ((64, 6144, 4160), 4), ((64, 6240, 4160), 2), ((128, 3072, 4160), 4),       # one round of 256
+    ((64, 4096, 4160), 4), ((64, 4096, 4032), 2),                               # 16 K steps in each of four
+    ((64, 4096, 2112), 2), ((64, 4096, 1984), 1),                               # ... of two
+    ((32, 12288, 4160), 2), ((16, 12288, 4160), 1),                             # int16 rows to 16 tokens, int8 to 32
+], ids=str)
+def test_where_byte_products_split_k(shape, splits):
+    query, (m, n, k) = _native.lib().rnsmx_packed_workspace_bytes, shape
+    rooms = {s: room(query, *shape, 6, plan=(10, 4, 1, 0, s, 0)) for s in (1, 2, 4)}
+    assert room(query, *shape, 6) == rooms[splits]
+    assert len(set(rooms.values())) == 3
+
+
 def runs_in(lib, mods, dtype, m, k, n, nbytes):
     """Whether a packed product accepts a workspace of nbytes.  Without a GPU a
     call that passes its checks ends at the launch, which reads nothing."""
