@@ -389,9 +389,10 @@ __device__ __forceinline__ int active_channels(KArgs<RCAP> &g, int64_t *red, int
       }
     });
     mx = wave_max_i64(mx);  // every lane holds the maximum
-    const int64_t best = static_cast<int64_t>(
-        (static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(mx) >> 32))) << 32) |
-        __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(mx)));
+    // readfirstlane returns a signed word: named as unsigned before they are joined
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(mx));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(mx) >> 32));
+    const int64_t best = static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
     const int64_t wmax = *g.w_absmax;
     int64_t bound;
     if (__builtin_mul_overflow(best, wmax, &bound)) bound = LLONG_MAX;
