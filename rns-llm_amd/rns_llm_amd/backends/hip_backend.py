@@ -112,13 +112,19 @@ class PreparedRNSWeight:
 
 @dataclass
 class RNSWorkspace:
-    """Reusable memory for one (rows, channels, stream) of one layer."""
+    """Reusable memory for one (rows, channels, stream) of one layer.
+
+    A call that needs more scratch than ``accumulators`` holds (another K,
+    weight form or plan) replaces it by a larger one.  Captured graphs hold
+    the address of the one they ran with, so it stays in ``replaced`` until
+    the workspace goes (each smaller than the next)."""
 
     accumulators: torch.Tensor  # uint8 scratch for the library
     output: torch.Tensor        # [M, N] int64
     channels: int
     m: int
     n: int
+    replaced: list = field(default_factory=list, repr=False, compare=False)
 
 
 class PreparedAdaptiveRNSWeight:
@@ -531,6 +537,7 @@ class HipRNSBackend:
             raise ValueError("bad workspace size")
         if workspace.accumulators.numel() < nbytes:
             # zero-filled for the arrival counters (see create_workspace)
+            workspace.replaced.append(workspace.accumulators)
             workspace.accumulators = torch.zeros(
                 (nbytes,), dtype=torch.uint8, device=workspace.output.device)
         return workspace.accumulators

@@ -110,3 +110,30 @@ def test_graph_replays_rnslinear_forward(backend, tokens):
             assert torch.equal(y, eager)
             want, _ = linear_oracle.linear_forward(x.cpu(), lin.weight.cpu(), lin.bias.cpu())
             assert torch.equal(y.cpu(), want)
+
+
+def test_a_graph_outlives_the_growth_of_its_workspace(backend):
+    """Two weights on one workspace: the second needs more scratch than the
+    captured call had.  The graph still runs, with the allocator's cache
+    emptied between (as entering a capture does), and writes to no tensor
+    that was allocated since."""
+    m, n = 70, 512
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    ints = lambda shape: torch.randint(-2000, 2001, shape, generator=gen, device=DEV, dtype=torch.int32).to(torch.int16)  # noqa: E731
+    weights, mods = [ints((n, k)) for k in (1024, 4096)], DENSE4 + (241, 239)
+    small, large = (backend.prepare_weight_nk(w, mods) for w in weights)
+    x, y = ints((m, 1024)), ints((m, 4096))
+    ws = backend.create_workspace(device=x.device, channels=6, m=m, n=n, k=1024)
+    graph, out = capture(lambda: backend.matmul_prepared_fused(x, small, workspace=ws))
+    before = ws.accumulators.data_ptr()
+    assert torch.equal(backend.matmul_prepared_fused(y, large, workspace=ws).double(), exact(y, weights[1]))
+    assert ws.accumulators.data_ptr() != before
+    torch.cuda.empty_cache()
+    others = [torch.full((1 << 20,), 7, dtype=torch.uint8, device=DEV) for _ in range(64)]
+    for _ in range(3):
+        x.copy_(ints((m, 1024)))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.double(), exact(x, weights[0]))
+        assert torch.equal(backend.matmul_prepared_fused(y, large, workspace=ws).double(), exact(y, weights[1]))
+        assert all(bool((t == 7).all()) for t in others)
