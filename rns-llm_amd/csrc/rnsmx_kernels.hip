@@ -1147,8 +1147,10 @@ static bool units_fit(const GemmChoice &c, const GemmArgs &g, bool araw) {
 // workgroups exceed four per CU (the residues they exchange then cost more
 // than the shorter steps save: 512 x 5120 x 2048 55 us against 46) and below
 // 17 rows, where the streaming kernels read the weight as fast.  The 5 %
-// between the estimates covers their error: over 180 shapes no product that
-// took units was slower by more than the timing's 2 %.
+// between the estimates covers most of their error: of 9707 products drawn
+// from 17 to 2500 rows, K 256 to 8192, N 256 to 16384, 5694 take units, in 0.67
+// of the other plan's time in the geometric mean; 15 of them are more than 5 %
+// slower than that plan, one of those more than 10 % (16 %).
 static bool units_auto(const GemmArgs &g, const GemmChoice &other, GemmChoice &c) {
   if (g.m <= 16) return false;
   auto rounds = [](int64_t workgroups) { return static_cast<double>((workgroups + 255) / 256); };
@@ -1174,12 +1176,18 @@ static bool units_auto(const GemmArgs &g, const GemmChoice &other, GemmChoice &c
     double base[4], step[4];
   } units[2] = {{2, 1, {8.5, 10, 11.5, 13}, {0.3, 0.3, 0.38, 0.58}},
                 {4, 2, {16.5, 20, 24, 28}, {0.3, 0.36, 0.75, 0.8}}};
+  // 32-row MFMA tiles past one round share their CUs, and a short K makes them
+  // cheaper than the estimate of two rounds
+  const bool shared = other.kind == kMfma && other.mb == 2 && tiles > 256 && tiles <= 512 && g.kp < 18 * 64;
   double best = 0.95 * before;
   bool found = false;
   for (const auto &u : units) {
     const GemmChoice t{kUnits, u.mb, u.nb, 0, 1, 0};
-    const int64_t per_cu = (gemm_grid(t, g.m, g.n).tiles * g.mods.channels + 255) / 256;
+    const int64_t groups = gemm_grid(t, g.m, g.n).tiles * g.mods.channels, per_cu = (groups + 255) / 256;
     if (per_cu > 4 || !units_fit(t, g, false)) continue;
+    // ... than large units of which a few start a second round (203 x 896 x 2757,
+    // 264 of them: 27.7 us against 22.5; 72 x 1008 x 5691: 28.3 against 23.5)
+    if (shared && u.mb == 4 && groups > 256 && groups <= 352) continue;
     const double now = u.base[per_cu - 1] + u.step[per_cu - 1] * steps;
     if (now < best) {
       best = now;

@@ -40,6 +40,9 @@ def room(query, m, n, k, channels, plan=None):
     ((64, 2304, 768, 5), (11, 2, 1, 0)), ((160, 1536, 1024, 6), (11, 2, 1, 0)),
     ((200, 515, 513, 6), (11, 2, 1, 0)), ((40, 12288, 4096, 6), (11, 4, 2, 0)),
     ((512, 768, 768, 6), None), ((300, 514, 576, 6), None), ((512, 12288, 4096, 6), None),
+    # 128 x 128 units of which a few start a second round, at 14, 16 and 17 K steps; 18 steps; more of them
+    ((203, 2757, 896, 6), None), ((72, 5691, 1008, 6), None), ((203, 2757, 1088, 6), None),
+    ((72, 5691, 1152, 6), (11, 4, 2, 0)), ((132, 4416, 1024, 6), (11, 4, 2, 0)),
     ((512, 2048, 5120, 6), None),                                                # past four workgroups per CU
 ], ids=str)
 def test_where_channel_units_are_taken(shape, units):
