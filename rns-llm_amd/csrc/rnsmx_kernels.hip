@@ -1434,13 +1434,33 @@ static GemmChoice bytes_auto(const GemmArgs &g, int ab) {
   return c;
 }
 
+// Whether a few int16 rows of k values take the channel rows `r` (packed_auto)
+// and not the byte rows.  Byte rows read the activations in place; rows that
+// are not 16-byte aligned cost them a copy, as the channel rows cost their
+// encode, and then the one block of channel rows is the shorter kernel (device
+// time, 4 x 2166 x 303 in 3 channels 6.7 us against 8.3, 1 x 7715 x 218 in 5 9.3
+// against 11.4; with two blocks it is even, 0.98).  Up to 4 channels and one
+// round of workgroups (N <= 4096), 9 to 16 such rows are 5 % faster as four blocks
+// (two fragments of byte rows), and from K = 1400 (2000 where nothing is copied) 17
+// to 32 rows as eight (four fragments: 27 x 4534 x 1781 22.7 us against 30.1, 27 x
+// 6272 x 302 28.7 against 35.1; past one round 0.43 to 0.9 of the channel rows').
+static bool channel_rows_win(const GemmArgs &g, const GemmChoice &r, int64_t k) {
+  if (r.kind != kRows) return false;
+  const bool copied = k % 8 != 0;
+  if (r.mb == 1) return copied;
+  if (g.mods.channels > 4 || g.n > 4096) return false;
+  return r.mb == 4 ? copied : r.mb == 8 && k >= (copied ? 1400 : 2000);
+}
+
 // a_dtype: the activations' type (-1: not known yet, any plan they could take).
-static int32_t packed_plan_from(const rnsmx_plan_t *plan, const GemmArgs &g, GemmChoice &c, int32_t a_dtype = -1) {
+static int32_t packed_plan_from(const rnsmx_plan_t *plan, const GemmArgs &g, GemmChoice &c, int64_t k = 0,
+                                int32_t a_dtype = -1) {
   if (plan == nullptr || plan->kind == kAuto) {
-    if ((a_dtype == RNSMX_INT8 || a_dtype == RNSMX_INT16) && bytes_fit(g))
-      c = bytes_auto(g, a_dtype == RNSMX_INT8 ? 1 : 2);
-    else
-      c = packed_auto(g);
+    c = packed_auto(g);
+    if ((a_dtype == RNSMX_INT8 || a_dtype == RNSMX_INT16) && bytes_fit(g)) {
+      const GemmChoice b = bytes_auto(g, a_dtype == RNSMX_INT8 ? 1 : 2);
+      if (a_dtype == RNSMX_INT8 || b.kind != kBytesRows || !channel_rows_win(g, c, k)) c = b;
+    }
     return RNSMX_OK;
   }
   if (plan->kind == kBytesRows || plan->kind == kBytesLds) {
@@ -1922,7 +1942,7 @@ static int32_t run_prepared(const void *a_dev, int32_t a_dtype, int32_t m, int32
   GemmArgs g = plan_args(m, n, k, R, araw);
   g.mods = *mods;
   GemmChoice c{};
-  if (int32_t rc = packed ? packed_plan_from(plan, g, c, a_dtype) : plan_from(plan, g, araw, true, c, true)) return rc;
+  if (int32_t rc = packed ? packed_plan_from(plan, g, c, k, a_dtype) : plan_from(plan, g, araw, true, c, true)) return rc;
   // a workspace made for more rows may hold no exchange area
   if (plan == nullptr || plan->kind == kAuto) {
     if (c.kind == kUnits && workspace_bytes < prepared_layout(araw, m, k, R, xchg_bytes(c, g)).total)

@@ -117,6 +117,20 @@ def test_sets_too_small_for_the_product(backend, moduli, m, dtype):
     assert torch.equal(run(backend, a, w, moduli, (10, 8, 1, 0, 2)), torch.from_numpy(r))
 
 
+# both sides of where a few int16 rows take the channel rows: rows that are
+# copied (K no multiple of 8) in one, two and four blocks; 17 to 32 rows from
+# K = 1400 or 2000; one column past one round of workgroups
+@pytest.mark.parametrize("m,k,n", [(4, 1001, 40), (5, 1001, 40), (12, 1001, 40), (4, 1000, 40), (12, 1000, 40), (17, 1396, 40),
+                                   (32, 1404, 40), (32, 1992, 40), (17, 2000, 40), (17, 2000, 4096), (17, 2000, 4097)])
+@pytest.mark.parametrize("channels", [3, 4, 6])
+def test_rows_on_both_sides_of_the_channel_rows(backend, m, k, n, channels):
+    moduli = DENSE6[:channels]
+    p = prod(moduli)
+    a, w, want = operands(m, k, n, torch.int16, m + k)
+    r = torch.remainder(want, p)
+    assert torch.equal(run(backend, a, w, moduli, None), torch.where(r > p >> 1, r - p, r))
+
+
 @pytest.mark.parametrize("m", [3, 40, 200])
 def test_adaptive_prefix(backend, m):
     a, w, want = operands(m, 512, 70, torch.int16, m)
