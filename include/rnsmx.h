@@ -247,7 +247,8 @@ int32_t rnsmx_matmul_prepared_fused(
  * afterwards.  No request may overlap staging_dev (RNSMX_EINVAL): rows are
  * copied there while others are still read.  Workspace as for that call.  One
  * launch for up to 16 int8 rows (4 channels, K a multiple of 16, 16-byte
- * aligned requests clear of out_dev).
+ * aligned requests clear of out_dev) unless the product splits a long K over
+ * workgroups.
  * Replaces the concatenation and product of matmul_prepared_fused_requests
  * (cuda_backend.py:647-703).
  */

@@ -2126,7 +2126,17 @@ int32_t rnsmx_matmul_requests(const void *const *requests, const int32_t *rows, 
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   int8_t *staging = static_cast<int8_t *>(staging_dev);
-  if (packed_form == 0 && in_place && n > 0 && request_rows_fits(m, k, *mods, a_dtype)) {
+  bool one_launch = packed_form == 0 && in_place && n > 0 && request_rows_fits(m, k, *mods, a_dtype);
+  if (one_launch && k >= 3072) {
+    // the one launch never splits K over workgroups; a product of few columns
+    // that does pays for the gather (device time): split in 8, 16 x 9648 x 702 12.9
+    // us in two launches against 19.4 in one, 15 x 15376 x 664 15.3 against 29.0;
+    // split in 4 once M K is large, 16 x 7824 x 629 12.7 against 16.7 but 4 x 7312
+    // x 1873 15.1 against 14.5
+    const GemmChoice c = auto_plan(plan_args(m, n, k, mods->channels, true), true, true);
+    one_launch = c.splits < 8 && (c.splits <= 1 || m * k <= 90112);
+  }
+  if (one_launch) {
     if (!packed_dev || !out_dev) return fail(RNSMX_EINVAL, "null tensor pointer");
     GemmArgs g = plan_args(m, n, k, mods->channels, true);
     g.mods = *mods;

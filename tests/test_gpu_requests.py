@@ -47,6 +47,24 @@ def test_merged_products(backend, rows, k, n, dtype, packed):
     assert torch.equal(torch.cat(clones), ws.fused.output)
 
 
+# a long K and few columns, on both sides of where the rows are gathered first
+# and the product splits K over workgroups
+@pytest.mark.parametrize("rows,k,n", [((5, 6), 8192, 100), ((5, 7), 8192, 100), ((16,), 5632, 300), ((16,), 5648, 300),
+                                      ((1, 3), 12288, 40), ((16,), 3072, 40)])
+def test_long_k(backend, rows, k, n):
+    gen = torch.Generator().manual_seed(k)
+    w = torch.randint(-127, 128, (n, k), generator=gen, dtype=torch.int32).to(torch.int8)
+    prepared = backend.prepare_weight_nk(w.cuda(), DENSE4)
+    ws = backend.create_request_batch_workspace(device=torch.device("cuda"), dtype=torch.int8, rows_per_request=rows, k=k,
+                                                channels=4, n=n)
+    for _ in range(2):
+        requests = [torch.randint(-128, 128, (r, k), generator=gen, dtype=torch.int32).to(torch.int8).cuda() for r in rows]
+        outs = backend.matmul_prepared_fused_requests(requests, prepared, workspace=ws)
+        assert torch.equal(ws.activations, torch.cat(requests))
+        for request, out in zip(requests, outs):
+            assert torch.equal(out.cpu(), exact(request, w))
+
+
 def test_refusals(backend):
     w = torch.ones((16, 64), dtype=torch.int8).cuda()
     prepared = backend.prepare_weight_nk(w, DENSE4)
