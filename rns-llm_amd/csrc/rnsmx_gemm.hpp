@@ -617,14 +617,25 @@ __device__ __forceinline__ void move_to_sgpr(double &v) {
   v = __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+// Lane `at`'s value of a vector double, in scalar registers.
+__device__ __forceinline__ double read_lane(double v, int at) {
+  const uint64_t w = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(w), at);
+  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(w >> 32), at);
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+
 // The rows of frac_sum for a prefix shorter than the set (adaptive calls):
 // from the bytes k_c with the roundings of the host's (frac_set); once per
-// wave.  x - h m is exact (h has 20 bits, m 8), so each row's rest is too.
-// Every channel's rows go to scalar registers before the next channel's are
-// formed: all at once, the divisions' registers would lower the occupancy of
-// the kernels that run this beside their first loads or their accumulators.
+// wave, lane c channel c (every lane is active here) and one lane more the
+// starting phase.  x - h m is exact (h has 20 bits, m 8), so each row's rest is
+// too.  One channel after the other, each with its own divisions, took a product
+// of up to 64 rows 0.46 us more at the median and 0.9 at most (250 adaptive
+// products of 6 to 30 us, 4 to 6 channels).
 template <int RCAP>
 __device__ __forceinline__ void prefix_frac(KArgs<RCAP> &g, Epi<RCAP> &e, int c_act) {
+  constexpr int kTurnLane = 7;
+  static_assert(RCAP < kTurnLane, "a lane per channel and one for the phase");
   uint32_t k0 = g.mods.kprefix[0][0], k1 = g.mods.kprefix[0][1];
   static_for<RCAP + 1>([&](auto I) {
     constexpr int i = decltype(I)::value;
@@ -633,29 +644,32 @@ __device__ __forceinline__ void prefix_frac(KArgs<RCAP> &g, Epi<RCAP> &e, int c_
       k1 = g.mods.kprefix[i][1];
     }
   });
-  static_for<RCAP>([&](auto C) {
-    constexpr int c = decltype(C)::value;
-    const uint32_t word = c < 4 ? k0 : k1;
-    double rest = static_cast<double>(static_cast<int8_t>((word >> (8 * (c % 4))) & 0xFFu));
-    const double m = static_cast<double>(max(g.mods.moduli[c], 1u));  // 0 past the set, whose k is 0
-    double scale = 1048576.0;
-    static_for<kFracParts<RCAP> - 1>([&](auto R) {
-      const double h = __builtin_rint(rest / m * scale) / scale;
-      e.f[decltype(R)::value][c] = h;
-      move_to_sgpr(e.f[decltype(R)::value][c]);
-      rest = __builtin_fma(-h, m, rest);
-      scale *= 1048576.0;
-    });
-    e.f[kFracParts<RCAP> - 1][c] = rest / m;
-    move_to_sgpr(e.f[kFracParts<RCAP> - 1][c]);
-  });
+  const int lane = static_cast<int>(threadIdx.x & 63);
   const int64_t p = prefix_at<RCAP>(g.mods, c_act);
   const double half = static_cast<double>((p - 1) >> 1);
   e.p = static_cast<double>(p);
-  e.turn = (half + 0.25) / e.p;
   e.magic = kRoundMagic - half;
+  uint32_t byte = 0, mod = 1;
+  static_for<RCAP>([&](auto C) {
+    constexpr int c = decltype(C)::value;
+    if (lane == c) {
+      byte = ((c < 4 ? k0 : k1) >> (8 * (c % 4))) & 0xFFu;
+      mod = max(g.mods.moduli[c], 1u);  // 0 past the set, whose k is 0
+    }
+  });
+  double rest = lane == kTurnLane ? half + 0.25 : static_cast<double>(static_cast<int8_t>(byte));
+  const double m = lane == kTurnLane ? e.p : static_cast<double>(mod);
+  double q = rest / m, scale = 1048576.0;
+  e.turn = read_lane(q, kTurnLane);
+  static_for<kFracParts<RCAP> - 1>([&](auto R) {
+    const double h = __builtin_rint(q * scale) / scale;
+    static_for<RCAP>([&](auto C) { e.f[decltype(R)::value][C] = read_lane(h, decltype(C)::value); });
+    rest = __builtin_fma(-h, m, rest);
+    scale *= 1048576.0;
+    q = rest / m;
+  });
+  static_for<RCAP>([&](auto C) { e.f[kFracParts<RCAP> - 1][C] = read_lane(q, decltype(C)::value); });
   move_to_sgpr(e.p);
-  move_to_sgpr(e.turn);
   move_to_sgpr(e.magic);
 }
 
@@ -1607,12 +1621,15 @@ __device__ __forceinline__ void stream_main(KArgs<RCAP> &g, const int c_act) {
   auto mfma_chunk = [&]() { mfma_part(std::integral_constant<int, 0>{}, std::integral_constant<int, U>{}); };
 
   Epi<RCAP> e;
-  if constexpr (kFrac<RCAP>) {
+  // a prefix's rows while the first chunk travels where its registers leave the
+  // occupancy as it is (4 channels), else ahead of it
+  constexpr bool kEarly = kFrac<RCAP> && RCAP != 4;
+  if constexpr (kEarly) {
     if (c_act != g.mods.channels) prefix_frac<RCAP>(g, e, c_act);
   }
   // first chunk in flight before the epilogue constants are waited for
   load_chunk(wave * U);
-  load_epi<RCAP, false>(g, e, c_act);
+  load_epi<RCAP, !kEarly>(g, e, c_act);
   pin_epi<RCAP>(e);
   int m_lim = g.m, n_lim = g.n;
   pin_sgpr(m_lim);
