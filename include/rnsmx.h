@@ -91,12 +91,18 @@ typedef struct rnsmx_moduli {
  * and packed weights; 128 x 128 tiles, 4- or 6-channel capacity, K a
  * multiple of 256; mb, nb, ks ignored; splits and tail as for kind 3), 9 and
  * 10 = packed weights by byte products (int8 and int16 activations, K up to
- * 65472, an activation byte plane below 4 GiB): 9 reads the activations as they are (up to mb = 1, 2 or 4 fragments
- * of 8 int16 or 16 int8 tokens, ks waves splitting K, never split), 10 runs
- * tiles of 16*mb x 24*mb (mb 4 or 8), split as kind 3.
+ * 65472, an activation byte plane below 4 GiB): 9 reads the activations as
+ * they are (up to mb = 1, 2 or 4 fragments of 8 int16 or 16 int8 tokens, ks
+ * waves splitting K, never split), 10 runs tiles of 16*mb x 24*mb (mb 4 or 8),
+ * split as kind 3.  11 = residue planes by channel units (5 or 6 channels, a
+ * plane below 4 GiB, tiles of 32*mb x 64*nb, 4 x 2 or 2 x 1): a workgroup
+ * computes one channel of a tile and the last of the channels reconstructs it
+ * from the residue bytes that the others left in the workspace; not for the
+ * no-allocation entry point.
  * splits: workgroups splitting K per output tile (0 or 1 = none; up to 4
- * channels, 6 for kind 8, and for the stream kernel ks = 1): each reduces its partial
- * sums to residues, and the last to finish a tile reconstructs it.  tail:
+ * channels, 6 for kinds 8 and 10, and for the stream kernel ks = 1): each
+ * reduces its partial sums to residues (kind 10: exact sums), and the last to
+ * finish a tile reconstructs it.  tail:
  * split only the tiles past the last full round of 256 (the others run
  * whole, first).  A plan
  * that names a kernel that is not built, or does not fit the call, makes the
@@ -384,18 +390,22 @@ int32_t rnsmx_matmul_packed_fused(
     void *out_dev, void *stream);
 
 /* The plan rnsmx_matmul_packed_fused chooses by itself for int32 activations
- * (host only); int8 and int16 ones take byte products (kinds 9 and 10). */
+ * (host only).  int8 and int16 ones take byte products (kinds 9 and 10) instead
+ * up to K = 65472, but for a few int16 rows that keep this plan's channel rows
+ * (kind 6) where those are shorter. */
 int32_t rnsmx_packed_plan(int64_t m, int64_t n, int64_t k, int32_t channels,
                           rnsmx_plan_t *out);
 
 /*
- * The plan rnsmx_matmul_prepared_fused chooses by itself for an M x N x K
- * product with `channels` moduli (kind 1-8, tile, ks, splits as in
- * rnsmx_plan_t).  raw_a != 0: int8 activations read in place, as the fused
- * entry points do for int8 sources with K a multiple of 16 whose
- * accumulators fit int32; 0: residue planes.  Host code only (no GPU call,
- * no stream).  No counterpart in the reference (cuBLAS picks its own
- * kernels there); for tests and tuning.
+ * The plan without channel units that rnsmx_matmul_prepared_fused chooses by
+ * itself for an M x N x K product with `channels` moduli (kind 1-8, tile, ks,
+ * splits as in rnsmx_plan_t).  raw_a != 0: int8 activations whose accumulators
+ * fit int32 (read in place, or from one padded copy where K is no multiple of
+ * 16); 0: residue planes, for which the call takes channel units (kind 11)
+ * instead where 5 or 6 channels of few tiles run faster so and the workspace
+ * has room for their exchange.  Host code only (no GPU call, no stream).  No
+ * counterpart in the reference (cuBLAS picks its own kernels there); for tests
+ * and tuning.
  */
 int32_t rnsmx_gemm_plan(int64_t m, int64_t n, int64_t k, int32_t channels,
                         int32_t raw_a, rnsmx_plan_t *out);
@@ -438,7 +448,10 @@ int64_t rnsmx_linear_workspace_bytes(int64_t rows, int64_t k, int64_t n,
  * [n] float32 or NULL; adaptive as in rnsmx_matmul_prepared_fused.  The
  * quantized activations, their scale and the GEMM scratch live in the
  * workspace (rnsmx_linear_workspace_bytes; the counter rule of the
- * conventions above applies).  Three launches, no host synchronisation.
+ * conventions above applies).  Up to 16 rows of 8 bits in 4 channels, up to the
+ * work where it pays, run in one launch (out_dev clear of x_dev); otherwise the
+ * quantizer's one or two launches come first, then the product's.  No host
+ * synchronisation; out_dev may overlap x_dev.
  * Replaces RNSLinear.forward's quantize -> backend -> dequantize chain
  * (src/rns_llm/layers/rns_linear.py:238-275) on a prepared weight.
  */

@@ -259,8 +259,9 @@ __global__ __launch_bounds__(256) void bytes_rows_kernel(const GemmArgsK<kBytesC
 // The column sums of the weight bytes are dot products on the VALU, beside the
 // MFMAs, one wave row taking even steps and the other odd ones.
 // K split: partial sums are doubles (exact integers), exchanged in two words
-// under the protocol of split_exchange; the row term is added by the first
-// split, the column sums by each for its own steps.
+// under the protocol of split_exchange: each split's column sums cover its own
+// steps, and the row term, of the whole K, is added once, by the wave that
+// finishes the tile.
 // K = 4096, N = 12288, 512 tokens (256 tiles of 128 x 192, one round): 87 us,
 // 2.4 POP/s of byte products, bound as lds_wide_kernel is by the staging and
 // the MFMAs together; the channel form's 2 R = 12 MFMAs per block took 312.

@@ -83,9 +83,9 @@ class Epilogue(ctypes.Structure):
 
 class Plan(ctypes.Structure):
     """Mirror of ``rnsmx_plan_t``: kind 0 = automatic; 1 stream, 2 MFMA,
-    3 LDS-staged, 4 wide stream, 5 three-wave MFMA, 6-8 and 9-10 as in
-    ``include/rnsmx.h``; tile blocks, ks, and the number of workgroups
-    splitting K."""
+    3 LDS-staged, 4 wide stream, 5 three-wave MFMA, 6 to 10 and 11 (channel
+    units) as in ``include/rnsmx.h``; tile blocks, ks, and the number of
+    workgroups splitting K."""
 
     _fields_ = [
         ("kind", ctypes.c_int32),

@@ -66,7 +66,9 @@ class PreparedRNSWeight:
     ``form == "planes"`` the P = R planes are the centered residues of every
     channel; with ``form == "packed"`` (int8/int16 weights, 2 bytes per value
     whatever R) the two planes are ``hi = v >> 8`` and ``lo = (v & 255) -
-    128`` and the kernels form each channel's residue from them.
+    128``: int8 and int16 activations multiply them byte by byte into the one
+    integer that every channel's residue belongs to, others into each
+    channel's residue.
     ``residues`` is the reference-shaped ``[R, K, N]`` tensor, unpacked on
     first access.
     """
@@ -970,10 +972,11 @@ class HipRNSBackend:
                                        workspace: RNSRequestBatchWorkspace | None = None,
                                        clone_outputs: bool = False) -> tuple[torch.Tensor, ...]:
         """Continuous batching (``cuda_backend.py:647-703``): the requests'
-        rows are stacked into one activation matrix (a single concatenation
-        into the staging buffer), multiplied in one fused call, and handed
-        back as row views of the merged output (copies with
-        ``clone_outputs``)."""
+        rows against one weight in one library call, which leaves them stacked
+        in the staging buffer (a few int8 rows are read where they lie, in one
+        launch), handed back as row views of the merged output (copies with
+        ``clone_outputs``).  Batches that the call does not take are
+        concatenated into the staging buffer first."""
         if len(requests) == 0:
             raise ValueError("no requests to batch")
         requests = tuple(requests)  # any sized container
